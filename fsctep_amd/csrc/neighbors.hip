@@ -10,9 +10,9 @@
 // so graph preparation's stable receiver sort keeps it.
 //
 // Steps: bounding box and grid (cells of side >= r where the cell budget allows), atoms bucketed by cell
-// (counting sort), 16 lanes per receiver counting its neighbours over the image points pos_j + s.cell
-// (the lanes split each cell's candidates), a scan into the receiver CSR (the caller reads the edge count),
-// then the same walk writing (src, s) keys, and a per-receiver rank sort of the keys.
+// (counting sort) with their positions in that order, one wave per receiver counting its neighbours over the
+// image points pos_j + s.cell, a scan into the receiver CSR (the caller reads the edge count), then the same
+// walk collecting the receiver's (src, s) keys in LDS, ranked there and written as edges.
 #include "common.h"
 #include "fsctep.h"
 #include "scan.h"
@@ -32,8 +32,19 @@ constexpr int KEY_IMAGES = 27;   // key = src * 27 + (sx+1)*9 + (sy+1)*3 + (sz+1
 __device__ __forceinline__ double dmul(double a, double b) { return __dmul_rn(a, b); }
 __device__ __forceinline__ double dadd(double a, double b) { return __dadd_rn(a, b); }
 
-__global__ __launch_bounds__(1024) void bbox_kernel(int64_t N, const double* __restrict__ pos, double* __restrict__ box) {
+// Block 0: the bounding box and the grid; the other blocks clear the cell counters (one launch for the three).
+// Grid dimensions G_k = max(1, floor(extent_k / r)) (so cells are at least r wide), halving the largest while
+// the product exceeds the cell budget.
+__global__ __launch_bounds__(1024) void grid_kernel(int64_t N, const double* __restrict__ pos, double r,
+                                                    int64_t cells_max, GridParams* __restrict__ g,
+                                                    int32_t* __restrict__ cnt) {
+  if (blockIdx.x > 0) {
+    for (int64_t i = (int64_t)(blockIdx.x - 1) * 1024 + threadIdx.x; i < cells_max; i += (int64_t)(gridDim.x - 1) * 1024)
+      cnt[i] = 0;
+    return;
+  }
   __shared__ double red[16][6];
+  __shared__ double box[6];
   double v[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
   for (int64_t i = threadIdx.x; i < N; i += 1024) {
 #pragma unroll
@@ -57,16 +68,12 @@ __global__ __launch_bounds__(1024) void bbox_kernel(int64_t N, const double* __r
   __syncthreads();
   if (threadIdx.x < 6) {
     const int k = threadIdx.x;
-    double r = red[0][k];
-    for (int w = 1; w < 16; ++w) r = k < 3 ? fmin(r, red[w][k]) : fmax(r, red[w][k]);
-    box[k] = r;
+    double v1 = red[0][k];
+    for (int w = 1; w < 16; ++w) v1 = k < 3 ? fmin(v1, red[w][k]) : fmax(v1, red[w][k]);
+    box[k] = v1;
   }
-}
-
-// One thread: grid dimensions G_k = max(1, floor(extent_k / r)) (so cells are at least r wide), halving the
-// largest while the product exceeds the cell budget.
-__global__ void grid_kernel(const double* __restrict__ box, double r, int64_t cells_max, GridParams* __restrict__ g) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
   int64_t G[3];
   for (int k = 0; k < 3; ++k) {
     double lo = box[k], hi = box[3 + k];
@@ -102,147 +109,196 @@ __device__ __forceinline__ int cell_coord(const GridParams& g, int k, double x) 
 
 __global__ __launch_bounds__(256) void assign_kernel(int64_t N, const double* __restrict__ pos,
                                                      const GridParams* __restrict__ gp, int32_t* __restrict__ atom_cell,
-                                                     int32_t* __restrict__ cnt) {
+                                                     int32_t* __restrict__ cnt, int32_t* __restrict__ slot) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= N) return;
   const GridParams g = *gp;
   const int c = (cell_coord(g, 0, pos[3 * i]) * g.G[1] + cell_coord(g, 1, pos[3 * i + 1])) * g.G[2] +
                 cell_coord(g, 2, pos[3 * i + 2]);
   atom_cell[i] = c;
-  atomicAdd(cnt + c, 1);
+  slot[i] = atomicAdd(cnt + c, 1);
 }
 
-__global__ __launch_bounds__(256) void place_kernel(int64_t N, const int32_t* __restrict__ atom_cell,
-                                                    const int32_t* __restrict__ cell_start, int32_t* __restrict__ cursor,
-                                                    int32_t* __restrict__ cell_atoms) {
+// Atoms and positions in cell order (unordered within a cell: the keys are ranked at the end).
+__global__ __launch_bounds__(256) void place_kernel(int64_t N, const double* __restrict__ pos,
+                                                    const int32_t* __restrict__ atom_cell,
+                                                    const int32_t* __restrict__ cell_start,
+                                                    const int32_t* __restrict__ slot, int32_t* __restrict__ cell_atoms,
+                                                    double* __restrict__ cell_pos) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= N) return;
-  const int32_t c = atom_cell[i];
-  cell_atoms[cell_start[c] + atomicAdd(cursor + c, 1)] = (int32_t)i;
+  const int64_t o = cell_start[atom_cell[i]] + slot[i];
+  cell_atoms[o] = (int32_t)i;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) cell_pos[3 * o + k] = pos[3 * i + k];
 }
 
 struct Walk {
-  const double* pos;
   const double* cell;   // [3][3], rows = lattice vectors
   const GridParams* grid;
   const int32_t* cell_start;
   const int32_t* cell_atoms;
+  const double* cell_pos;   // positions in the order of cell_atoms
   int64_t N;
   int32_t pbc[3];
   double r2, reach;     // r^2 for the test; r (1 + 1e-9) for the cell range
 };
 
-// A group of RL = 16 consecutive lanes per receiver j (four receivers per wave) visits every (i, s) within
-// r of j (see the file comment).  The loops over the image shifts and the cells in range are uniform in
-// the group; its lanes split each cell's atoms (16 candidates per step, about a cell's content at the
-// benchmark densities), and a step's hits are numbered in lane order by a ballot and a prefix popcount
-// over the group's bits.  For each step with hits, f(hit, i, key, rank, count) is called by every lane of
-// the group (hit: this lane's candidate is a neighbour; rank: its position among the receiver's hits so
-// far; count: the step's hits).  Returns the number visited (the same in every lane of the group).
-constexpr int RL = 16;
+// One wave visits every (i, s) within r of the receiver j at place p of the cell order (see the file
+// comment).  The loops over the image shifts and the cell columns in range are uniform in the wave.  The cells
+// of a column (consecutive along z) are consecutive in the cell order, so a column's candidates are one run,
+// taken 64 at a time (about 40 in the three cells of side 5 at 0.1 atoms per cubic unit; a cell alone holds
+// 13); the lanes test the images against the box at once, which leaves one to eight to walk.  A step's hits
+// are numbered in lane order by a ballot and a prefix popcount; f(hit, key, rank) is called by every lane
+// for each step with hits (rank: the hit's position among the receiver's hits so far).  Returns the number
+// visited.  Count and fill at 10,000 atoms and 52 neighbours: 28 and 39 us (70 and 97 us with 16 lanes per
+// receiver, cell by cell, and the keys through memory to a rank kernel); bound by the fp64 arithmetic of the
+// candidates and the latency of nine columns one after the other.
 template <typename F>
-__device__ __forceinline__ int32_t walk_receiver_wave(const Walk& w, int64_t j, int lane, F&& f) {
-  const int sub = lane & (RL - 1), gshift = lane & ~(RL - 1);
-  const GridParams g = *w.grid;
-  const double pj[3] = {w.pos[3 * j], w.pos[3 * j + 1], w.pos[3 * j + 2]};
-  double a[9];
+__device__ __forceinline__ int32_t walk_receiver(const Walk& w, int64_t p0, int lane, F&& f) {
+  const GridParams& g = *w.grid;
+  const int32_t j = w.cell_atoms[p0];
+  const double pj[3] = {w.cell_pos[3 * p0], w.cell_pos[3 * p0 + 1], w.cell_pos[3 * p0 + 2]};
+  const uint64_t below = lane ? (~0ull >> (64 - lane)) : 0ull;
+  const auto image = [&](int code, double* sv, double* p) {   // image code's shift and the receiver's image point
+    const double s0 = code / 9 - 1, s1 = (code / 3) % 3 - 1, s2 = code % 3 - 1;
 #pragma unroll
-  for (int t = 0; t < 9; ++t) a[t] = w.cell[t];
-  const uint64_t below = sub ? (~0ull >> (64 - sub)) : 0ull;
+    for (int k = 0; k < 3; ++k) {
+      sv[k] = dadd(dadd(dmul(s0, w.cell[k]), dmul(s1, w.cell[3 + k])), dmul(s2, w.cell[6 + k]));
+      p[k] = pj[k] + sv[k];
+    }
+  };
+  // lane c tests image c: no atom lies outside [lo, hi], so an image point farther than r from the box has no
+  // neighbours (a non-finite one neither)
+  uint64_t images;
+  {
+    const int code = lane < KEY_IMAGES ? lane : 0;
+    bool on = lane < KEY_IMAGES && abs(code / 9 - 1) <= w.pbc[0] && abs((code / 3) % 3 - 1) <= w.pbc[1] &&
+              abs(code % 3 - 1) <= w.pbc[2];
+    double sv[3], p[3];
+    image(code, sv, p);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      if (!(p[k] == p[k]) || p[k] + w.reach < g.lo[k] || p[k] - w.reach > g.hi[k]) on = false;
+    images = __ballot(on);
+  }
   int32_t n = 0;
-  for (int sx = -w.pbc[0]; sx <= w.pbc[0]; ++sx)
-    for (int sy = -w.pbc[1]; sy <= w.pbc[1]; ++sy)
-      for (int sz = -w.pbc[2]; sz <= w.pbc[2]; ++sz) {
-        double sv[3], p[3];
-        int clo[3], chi[3];
-        bool empty = false;
+  for (; images; images &= images - 1) {
+    const int code = __ffsll((unsigned long long)images) - 1;
+    double sv[3], p[3];
+    image(code, sv, p);
+    int clo[3], chi[3];
 #pragma unroll
-        for (int k = 0; k < 3; ++k) {
-          sv[k] = dadd(dadd(dmul((double)sx, a[k]), dmul((double)sy, a[3 + k])), dmul((double)sz, a[6 + k]));
-          p[k] = pj[k] + sv[k];
-          // no atom lies outside [lo, hi]: an image point farther than r from the box has no neighbours
-          if (p[k] + w.reach < g.lo[k] || p[k] - w.reach > g.hi[k]) empty = true;
-          clo[k] = cell_coord(g, k, p[k] - w.reach);
-          chi[k] = cell_coord(g, k, p[k] + w.reach);
-        }
-        if (empty || !(p[0] == p[0] && p[1] == p[1] && p[2] == p[2])) continue;
-        const int code = (sx + 1) * 9 + (sy + 1) * 3 + (sz + 1);
-        const bool self_image = sx == 0 && sy == 0 && sz == 0;
-        for (int cx = clo[0]; cx <= chi[0]; ++cx)
-          for (int cy = clo[1]; cy <= chi[1]; ++cy)
-            for (int cz = clo[2]; cz <= chi[2]; ++cz) {
-              const int c = (cx * g.G[1] + cy) * g.G[2] + cz;
-              const int32_t qb = w.cell_start[c], qe = w.cell_start[c + 1];
-              for (int32_t q0 = qb; q0 < qe; q0 += RL) {
-                const int32_t q = q0 + sub;
-                bool hit = false;
-                int32_t i = 0;
-                if (q < qe) {
-                  i = w.cell_atoms[q];
-                  if (!(self_image && i == j)) {
-                    const double dx = dadd(pj[0] - w.pos[3 * (int64_t)i], sv[0]);
-                    const double dy = dadd(pj[1] - w.pos[3 * (int64_t)i + 1], sv[1]);
-                    const double dz = dadd(pj[2] - w.pos[3 * (int64_t)i + 2], sv[2]);
-                    const double d2 = dadd(dadd(dmul(dx, dx), dmul(dy, dy)), dmul(dz, dz));
-                    hit = d2 < w.r2;
-                  }
-                }
-                // this group's bits of the ballot of the lanes still in the loop
-                const uint64_t mask = (__ballot(hit) >> gshift) & ((1ull << RL) - 1);
-                if (mask) {
-                  const int cnt = __popcll(mask);
-                  f(hit, i, (int64_t)i * KEY_IMAGES + code, n + __popcll(mask & below), cnt);
-                  n += cnt;
-                }
-              }
-            }
+    for (int k = 0; k < 3; ++k) {
+      clo[k] = cell_coord(g, k, p[k] - w.reach);
+      chi[k] = cell_coord(g, k, p[k] + w.reach);
+    }
+    const bool self_image = code == KEY_IMAGES / 2;
+    const int ny = chi[1] - clo[1] + 1, ncol = (chi[0] - clo[0] + 1) * ny;
+    for (int c0 = 0; c0 < ncol; c0 += 64) {
+      // lane c holds the bounds of column c0 + c
+      const int col = c0 + lane;
+      int32_t qb_l = 0, qe_l = 0;
+      if (col < ncol) {
+        const int c = ((clo[0] + col / ny) * g.G[1] + clo[1] + col % ny) * g.G[2];
+        qb_l = w.cell_start[c + clo[2]];
+        qe_l = w.cell_start[c + chi[2] + 1];
       }
+      const int nc = ncol - c0 < 64 ? ncol - c0 : 64;
+      for (int cc = 0; cc < nc; ++cc) {
+        const int32_t qb = __builtin_amdgcn_readlane(qb_l, cc), qe = __builtin_amdgcn_readlane(qe_l, cc);
+        for (int32_t q0 = qb; q0 < qe; q0 += 64) {
+          const int32_t q = q0 + lane;
+          bool hit = false;
+          int32_t i = 0;
+          if (q < qe) {
+            i = w.cell_atoms[q];
+            const double dx = dadd(pj[0] - w.cell_pos[3 * (int64_t)q], sv[0]);
+            const double dy = dadd(pj[1] - w.cell_pos[3 * (int64_t)q + 1], sv[1]);
+            const double dz = dadd(pj[2] - w.cell_pos[3 * (int64_t)q + 2], sv[2]);
+            const double d2 = dadd(dadd(dmul(dx, dx), dmul(dy, dy)), dmul(dz, dz));
+            hit = d2 < w.r2 && !(self_image && i == j);
+          }
+          const uint64_t mask = __ballot(hit);
+          if (mask) {
+            f(hit, (int64_t)i * KEY_IMAGES + code, n + __popcll(mask & below));
+            n += __popcll(mask);
+          }
+        }
+      }
+    }
+  }
   return n;
 }
 
+// Four receivers per block, in cell order: the waves that run together read the same cells.
 __global__ __launch_bounds__(256) void count_kernel(Walk w, int32_t* __restrict__ deg) {
-  const int64_t j = (int64_t)blockIdx.x * (256 / RL) + threadIdx.x / RL;
-  if (j >= w.N) return;   // uniform in the lane group
+  const int64_t p = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (p >= w.N) return;
   const int lane = threadIdx.x & 63;
-  const int32_t n = walk_receiver_wave(w, j, lane, [](bool, int32_t, int64_t, int32_t, int) {});
-  if ((lane & (RL - 1)) == 0) deg[j] = n;
+  const int32_t n = walk_receiver(w, p, lane, [](bool, int64_t, int32_t) {});
+  if (lane == 0) deg[w.cell_atoms[p]] = n;
 }
 
-__global__ __launch_bounds__(256) void fill_kernel(Walk w, const int32_t* __restrict__ dst_ptr, int64_t E,
-                                                   int64_t* __restrict__ keys, int32_t* __restrict__ key_dst) {
-  const int64_t j = (int64_t)blockIdx.x * (256 / RL) + threadIdx.x / RL;
-  if (j >= w.N) return;   // uniform in the lane group
-  const int lane = threadIdx.x & 63;
-  const int64_t beg = dst_ptr[j], end = dst_ptr[j + 1];
-  walk_receiver_wave(w, j, lane, [&](bool hit, int32_t, int64_t key, int32_t rank, int) {
-    const int64_t o = beg + rank;
-    if (hit && o < end && o < E) {   // the counts came from the same walk: never false, kept as a bound
-      keys[o] = key;
-      key_dst[o] = (int32_t)j;
-    }
-  });
-}
+constexpr int KEY_CAP = 512;   // neighbours of a receiver whose keys are ranked in LDS (as 32-bit keys)
 
-// Final order: each key's rank within its receiver's slots.
-__global__ __launch_bounds__(256) void rank_kernel(int64_t N, int64_t E, const int32_t* __restrict__ dst_ptr,
-                                                   const int64_t* __restrict__ keys, const int32_t* __restrict__ key_dst,
-                                                   int64_t* __restrict__ edge_src, int64_t* __restrict__ edge_dst,
-                                                   double* __restrict__ edge_shifts) {
-  const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (p >= E) return;
-  const int64_t key = keys[p];
-  const int32_t j = key_dst[p];
-  if (j < 0 || j >= N) return;   // every slot is written by fill_kernel; kept as a bound
-  const int32_t a = dst_ptr[j], b = dst_ptr[j + 1];
-  int32_t rank = 0;
-  for (int32_t q = a; q < b; ++q) rank += keys[q] < key;
-  const int64_t o = a + rank;
-  const int code = (int)(key % KEY_IMAGES);
-  edge_src[o] = key / KEY_IMAGES;
+__device__ __forceinline__ void write_edge(int64_t o, int64_t key, int64_t j, int64_t* __restrict__ edge_src,
+                                           int64_t* __restrict__ edge_dst, double* __restrict__ edge_shifts) {
+  const int64_t i = key / KEY_IMAGES;
+  const int code = (int)(key - i * KEY_IMAGES);
+  edge_src[o] = i;
   edge_dst[o] = j;
   edge_shifts[3 * o] = (double)(code / 9 - 1);
   edge_shifts[3 * o + 1] = (double)((code / 3) % 3 - 1);
   edge_shifts[3 * o + 2] = (double)(code % 3 - 1);
+}
+
+// Keys of one receiver per wave, then each key's rank among them, which is its place in the receiver's
+// segment.  Up to KEY_CAP keys that fit 32 bits (159 million atoms) stay in LDS, padded with the largest key
+// so that they are compared four at a time; the others go through `keys` and are read back past the L1 (the
+// segments of other receivers share cache lines).
+__global__ __launch_bounds__(256) void fill_kernel(Walk w, const int32_t* __restrict__ dst_ptr, int64_t E, int64_t* keys,
+                                                   int64_t* __restrict__ edge_src, int64_t* __restrict__ edge_dst,
+                                                   double* __restrict__ edge_shifts) {
+  __shared__ uint4 lkeys[4][KEY_CAP / 4];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t p = (int64_t)blockIdx.x * 4 + wave;
+  if (p >= w.N) return;   // no barrier below: each wave works on its own keys
+  const int lane = threadIdx.x & 63;
+  const int64_t j = w.cell_atoms[p];
+  const int64_t beg = dst_ptr[j], end = dst_ptr[j + 1] < E ? dst_ptr[j + 1] : E;
+  const int32_t deg = (int32_t)(end - beg);
+  // the counts came from the same walk, so rank < deg always holds: kept as a bound
+  if (deg <= KEY_CAP && w.N < (int64_t)(UINT32_MAX / KEY_IMAGES)) {
+    uint32_t* mine = reinterpret_cast<uint32_t*>(lkeys[wave]);
+    if (lane < 4 && (deg & ~3) + lane < KEY_CAP) mine[(deg & ~3) + lane] = UINT32_MAX;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    walk_receiver(w, p, lane, [&](bool hit, int64_t key, int32_t rank) {
+      if (hit && rank < deg) mine[rank] = (uint32_t)key;
+    });
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    for (int32_t t = lane; t < deg; t += 64) {
+      const uint32_t key = mine[t];
+      int32_t rank = 0;
+      for (int32_t q = 0; 4 * q < deg; ++q) {
+        const uint4 o = lkeys[wave][q];
+        rank += (o.x < key) + (o.y < key) + (o.z < key) + (o.w < key);
+      }
+      write_edge(beg + rank, key, j, edge_src, edge_dst, edge_shifts);
+    }
+  } else {
+    walk_receiver(w, p, lane, [&](bool hit, int64_t key, int32_t rank) {
+      if (hit && rank < deg) __hip_atomic_store(keys + beg + rank, key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    });
+    __threadfence();
+    for (int32_t t = lane; t < deg; t += 64) {
+      const int64_t key = __hip_atomic_load(keys + beg + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      int32_t rank = 0;
+      for (int32_t q = 0; q < deg; ++q)
+        rank += __hip_atomic_load(keys + beg + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < key;
+      write_edge(beg + rank, key, j, edge_src, edge_dst, edge_shifts);
+    }
+  }
 }
 
 int64_t cells_budget(int64_t N) {
@@ -251,7 +307,7 @@ int64_t cells_budget(int64_t N) {
 }
 
 struct NbrWs {
-  int64_t cnt, cur, grid, box, cell_start, tot, atom_cell, cell_atoms, deg, total, cells, nb;
+  int64_t cnt, grid, cell_pos, cell_start, tot, atom_cell, cell_atoms, deg, total, cells, nb;
 };
 
 NbrWs nbr_ws(int64_t N) {
@@ -260,10 +316,9 @@ NbrWs nbr_ws(int64_t N) {
   w.nb = (w.cells + 1 + SCAN_TILE - 1) / SCAN_TILE;
   int64_t o = 0;
   w.cnt = o;        o += w.cells;
-  w.cur = o;        o += w.cells;   // the zero-filled prefix ends here
   o = (o + 1) & ~int64_t(1);        // 8-byte alignment of the double fields
   w.grid = o;       o += (int64_t)(sizeof(GridParams) / 4);
-  w.box = o;        o += 12;
+  w.cell_pos = o;   o += 6 * N;
   w.cell_start = o; o += w.cells + 1;
   w.tot = o;        o += w.nb;
   w.atom_cell = o;  o += N;
@@ -273,14 +328,13 @@ NbrWs nbr_ws(int64_t N) {
   return w;
 }
 
-Walk make_walk(int64_t N, const double* pos, const double* cell, const int32_t* pbc, double cutoff, int32_t* ws,
-               const NbrWs& w) {
+Walk make_walk(int64_t N, const double* cell, const int32_t* pbc, double cutoff, int32_t* ws, const NbrWs& w) {
   Walk k;
-  k.pos = pos;
   k.cell = cell;
   k.grid = reinterpret_cast<const GridParams*>(ws + w.grid);
   k.cell_start = ws + w.cell_start;
   k.cell_atoms = ws + w.cell_atoms;
+  k.cell_pos = reinterpret_cast<const double*>(ws + w.cell_pos);
   k.N = N;
   for (int a = 0; a < 3; ++a) k.pbc[a] = pbc[a] ? 1 : 0;
   k.r2 = cutoff * cutoff;
@@ -312,29 +366,27 @@ int fsc_neighbor_count(int64_t n_nodes, const double* pos, const double* cell, c
   const int64_t N = n_nodes;
   const NbrWs w = nbr_ws(N);
   int32_t* ws = workspace;
-  fill_i32_kernel<<<grid_of(w.cur + w.cells) < 1024 ? grid_of(w.cur + w.cells) : 1024, 256, 0, stream>>>(
-      ws, w.cur + w.cells, 0);
   if (N == 0) {
     fill_i32_kernel<<<1, 256, 0, stream>>>(dst_ptr, 1, 0);
     return check_launch("fsc_neighbor_count") ? 2 : 0;
   }
-  double* box = reinterpret_cast<double*>(ws + w.box);
   GridParams* gp = reinterpret_cast<GridParams*>(ws + w.grid);
-  bbox_kernel<<<1, 1024, 0, stream>>>(N, pos, box);
-  grid_kernel<<<1, 64, 0, stream>>>(box, cutoff, w.cells, gp);
-  assign_kernel<<<grid_of(N), 256, 0, stream>>>(N, pos, gp, ws + w.atom_cell, ws + w.cnt);
+  const int64_t fill_blocks = (w.cells + 4095) / 4096;
+  grid_kernel<<<(unsigned)(1 + (fill_blocks < 255 ? fill_blocks : 255)), 1024, 0, stream>>>(N, pos, cutoff, w.cells, gp,
+                                                                                           ws + w.cnt);
+  int32_t* slot = ws + w.deg;   // the degrees come later
+  assign_kernel<<<grid_of(N), 256, 0, stream>>>(N, pos, gp, ws + w.atom_cell, ws + w.cnt, slot);
   ScanArgs sa;
   sa.cnt[0] = sa.cnt[1] = ws + w.cnt;
   sa.out[0] = sa.out[1] = ws + w.cell_start;
   sa.tot[0] = sa.tot[1] = ws + w.tot;
   sa.n = w.cells;
   FSC_CHECK_ARG(w.nb <= SCAN_MAX_BLOCKS, "fsc_neighbor_count: too many cells for the scan");
-  scan_blocks_kernel<<<dim3((unsigned)w.nb, 1), SCAN_T, 0, stream>>>(sa);
-  scan_totals_kernel<<<dim3(1, 1), 1024, 0, stream>>>(sa, (int)w.nb);
-  scan_add_kernel<<<dim3((unsigned)w.nb, 1), SCAN_T, 0, stream>>>(sa);
-  place_kernel<<<grid_of(N), 256, 0, stream>>>(N, ws + w.atom_cell, ws + w.cell_start, ws + w.cur, ws + w.cell_atoms);
-  const Walk walk = make_walk(N, pos, cell, pbc, cutoff, ws, w);
-  count_kernel<<<(unsigned)((N + 256 / RL - 1) / (256 / RL)), 256, 0, stream>>>(walk, ws + w.deg);
+  launch_scan(sa, 1, stream);
+  place_kernel<<<grid_of(N), 256, 0, stream>>>(N, pos, ws + w.atom_cell, ws + w.cell_start, slot, ws + w.cell_atoms,
+                                               reinterpret_cast<double*>(ws + w.cell_pos));
+  const Walk walk = make_walk(N, cell, pbc, cutoff, ws, w);
+  count_kernel<<<(unsigned)((N + 3) / 4), 256, 0, stream>>>(walk, ws + w.deg);
   // receiver CSR: exclusive scan of the degrees into dst_ptr[0..N]
   const int64_t nbn = (N + 1 + SCAN_TILE - 1) / SCAN_TILE;
   FSC_CHECK_ARG(nbn <= SCAN_MAX_BLOCKS, "fsc_neighbor_count: too many nodes for the scan");
@@ -343,9 +395,7 @@ int fsc_neighbor_count(int64_t n_nodes, const double* pos, const double* cell, c
   sd.out[0] = sd.out[1] = dst_ptr;
   sd.tot[0] = sd.tot[1] = ws + w.cnt;   // the cell counts are dead once cell_start is built
   sd.n = N;
-  scan_blocks_kernel<<<dim3((unsigned)nbn, 1), SCAN_T, 0, stream>>>(sd);
-  scan_totals_kernel<<<dim3(1, 1), 1024, 0, stream>>>(sd, (int)nbn);
-  scan_add_kernel<<<dim3((unsigned)nbn, 1), SCAN_T, 0, stream>>>(sd);
+  launch_scan(sd, 1, stream);
   return check_launch("fsc_neighbor_count") ? 2 : 0;
 }
 
@@ -359,10 +409,8 @@ int fsc_neighbor_fill(int64_t n_nodes, int64_t n_edges, const double* pos, const
   const int64_t N = n_nodes, E = n_edges;
   const NbrWs w = nbr_ws(N);
   int64_t* keys = reinterpret_cast<int64_t*>(fill_ws);   // 2E int32, 8-byte aligned by the caller
-  int32_t* key_dst = fill_ws + 2 * E;
-  const Walk walk = make_walk(N, pos, cell, pbc, cutoff, workspace, w);
-  fill_kernel<<<(unsigned)((N + 256 / RL - 1) / (256 / RL)), 256, 0, stream>>>(walk, dst_ptr, E, keys, key_dst);
-  rank_kernel<<<grid_of(E), 256, 0, stream>>>(N, E, dst_ptr, keys, key_dst, edge_src, edge_dst, edge_shifts);
+  const Walk walk = make_walk(N, cell, pbc, cutoff, workspace, w);
+  fill_kernel<<<(unsigned)((N + 3) / 4), 256, 0, stream>>>(walk, dst_ptr, E, keys, edge_src, edge_dst, edge_shifts);
   return check_launch("fsc_neighbor_fill") ? 2 : 0;
 }
 

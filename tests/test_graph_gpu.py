@@ -198,3 +198,17 @@ def test_conv_results_do_not_depend_on_the_node_order():
             fld = torch.tensor(bench._field(1, w["seed"]), dtype=torch.float32, device=DEV)
             r0, r1 = (energy_forces(model, pos, batch, cell, g, external_tensor=fld)[:2] for g in (g0, g1))
         assert torch.equal(r0[0], r1[0]) and torch.equal(r0[1], r1[1]), mode
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,E", [(8191, 20000), (8192, 20000), (16383, 30000), (16384, 30011), (20000, 30011)])
+def test_graph_prepare_around_the_scan_sizes(N, E):
+    """One step, several steps and the three-pass form of the CSR scan, on receiver-sorted edges with runs longer
+    than a wave (one atomic per run) and on the same edges shuffled."""
+    src, dst, species = _graph(N, E, 5, N, hub=11)
+    dst[E // 2:] = np.sort(dst[E // 2:])
+    g, sh = _run(src, dst, species, 5)
+    _check(src, dst, species, 5, g, sh)
+    p = np.random.default_rng(0).permutation(E)
+    g, sh = _run(src[p], dst[p], species, 5)
+    _check(src[p], dst[p], species, 5, g, sh)

@@ -118,3 +118,15 @@ def test_feeds_graph_preparation_unchanged():
     src, dst, sh, _ = [torch.as_tensor(a).to(DEV) for a in _gpu(s.pos, s.cell, 5.0)]
     g = prepare_graph(src, dst, sh, 1000)
     assert torch.equal(g.order.cpu(), torch.arange(src.shape[0], dtype=torch.int32))
+
+
+@pytest.mark.parametrize("n,r", [(513, 9.0), (514, 9.0), (700, 9.0), (700, 3.2)])
+def test_receivers_around_the_key_capacity(n, r):
+    """512 neighbours rank their keys in LDS, more go through memory; the last case mixes both in one list."""
+    rng = np.random.default_rng(n)
+    pos = rng.uniform(0.0, 5.0, (n, 3))
+    cell = np.eye(3) * 100.0
+    got = _gpu(pos, cell, r, pbc=False)
+    _equal(got, _brute(pos, cell, r, (0, 0, 0)), n)
+    deg = np.diff(got[3])
+    assert deg.max() == n - 1 if r > 8.7 else (deg.max() > 512 and deg.min() < 512)
