@@ -259,17 +259,119 @@ __global__ __launch_bounds__(256) void project_t_kernel(Dims d, const T* __restr
   }
 }
 
-// out[idx] (+)= sum over parts of part[p][idx], parts in order.
-template <typename T>
-__global__ void sum_parts_kernel(int64_t n, int nparts, const T* __restrict__ part, T* __restrict__ out, int acc) {
-  for (int64_t idx = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; idx < n; idx += (int64_t)gridDim.x * blockDim.x) {
-    T s = 0;
-    for (int p = 0; p < nparts; ++p) s += part[(int64_t)p * n + idx];
-    put(out + idx, s, acc);
+// grad_v alone: grad_v[b][n] (+)= sum_{m,pk} U[m*m2+n][pk] T_b[m][pk].  One wave per element forms T_b on the
+// matrix cores (rows m padded to 16, NT tiles of 16 columns pk, K = channels), so gy and a are read once from
+// global memory and nothing but U is staged; the general kernel above moves both through LDS and keeps one lane
+// a column busy.  The lane's partial sums of the m2 outputs are added over the wave by halving exchanges (8
+// outputs: 4 + 2 + 1 + 3 shuffles).  60,011 elements, 128 channels, m1 7, PK 7 (0.43 GB read): 440 -> 110 us on
+// average over the lmax 3 buckets, 4 TB/s.  Channels in whole 4-vectors: I % 4 == 0, 16-byte aligned gy.
+template <typename T, int NT>
+__global__ __launch_bounds__(256) void project_tv_kernel(Dims d, const T* __restrict__ gy, const T* __restrict__ a,
+                                                         const T* __restrict__ U, T* __restrict__ grad_v, int acc) {
+  using M = Mma<T>;
+  using V = typename M::V;
+  extern __shared__ __align__(16) char smraw[];
+  T* us = reinterpret_cast<T*>(smraw);   // [m2][16][16*NT], zero past m1 and PK
+  const int PK = d.P * d.K;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, q = lane >> 4;
+  for (int idx = threadIdx.x; idx < d.m2 * 256 * NT; idx += 256) {
+    const int pk = idx % (16 * NT), nm = idx / (16 * NT), m = nm & 15, n = nm >> 4;
+    us[idx] = (m < d.m1 && pk < PK) ? U[(m * d.m2 + n) * PK + pk] : T(0);
+  }
+  __syncthreads();
+  const bool rv = r < d.m1;
+  for (int64_t b = (int64_t)blockIdx.x * 4 + wave; b < d.B; b += (int64_t)gridDim.x * 4) {
+    V t[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) t[j] = M::zero();
+    const T* ab = a + b * d.I * d.m1 + (rv ? r : 0);
+    const T* gb = gy + b * PK * d.I;
+#pragma unroll 2
+    for (int i0 = 0; i0 < d.I; i0 += 16) {
+      const bool iv = i0 + 4 * q < d.I;   // the channel tail enters as zeros on both sides
+      const int ic = iv ? i0 + 4 * q : 0;
+      V av, bv[NT];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) av[s] = ab[(ic + s) * d.m1];
+#pragma unroll
+      for (int j = 0; j < NT; ++j) bv[j] = M::ld(gb + (int64_t)min(16 * j + r, PK - 1) * d.I + ic);
+#pragma unroll
+      for (int s = 0; s < 4; ++s) av[s] = iv && rv ? av[s] : T(0);
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) bv[j][s] = iv ? bv[j][s] : T(0);
+        t[j] = M::mma(av, bv[j], t[j]);
+      }
+    }
+    for (int n0 = 0; n0 < d.m2; n0 += 8) {
+      T s[8];
+#pragma unroll
+      for (int n = 0; n < 8; ++n) {
+        s[n] = 0;
+        if (n0 + n < d.m2) {
+          const T* un = us + (n0 + n) * 256 * NT + r;
+#pragma unroll
+          for (int jj = 0; jj < 4; ++jj)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+              const T uv = un[M::row(q, jj) * 16 * NT + 16 * j];
+              // rows past m1 hold 0 * gy and columns past PK repeat column PK - 1: left out, not multiplied
+              // by zero, so that an infinite input stays in its own sums
+              s[n] += (M::row(q, jj) < d.m1 && 16 * j + r < PK) ? uv * t[j][jj] : T(0);
+            }
+        }
+      }
+#pragma unroll
+      for (int k = 4; k > 0; k >>= 1) {   // lane bits 5, 4, 3 choose the half of the outputs it keeps
+        const int off = 8 * k;
+        const bool hi = lane & off;
+#pragma unroll
+        for (int n = 0; n < 4; ++n)
+          if (n < k) {
+            const T mine = hi ? s[n + k] : s[n], other = hi ? s[n] : s[n + k];
+            s[n] = mine + __shfl_xor(other, off, 64);
+          }
+      }
+#pragma unroll
+      for (int off = 4; off > 0; off >>= 1) s[0] += __shfl_xor(s[0], off, 64);
+      const int n = n0 + (lane >> 3);
+      if ((lane & 7) == 0 && n < d.m2) put(grad_v + b * d.m2 + n, s[0], acc);
+    }
   }
 }
 
-// ---------------------------------------------------------------- channel mix (MFMA)
+// out[idx] (+)= sum over parts of part[p][idx], in a fixed order: 8 groups of threads take every eighth part,
+// their sums are added in order.  A thread per output walked up to 4096 parts one load after another in 64
+// blocks (P O I = 16,384 outputs, 2048 parts: 282 us); 32 outputs a block keep 128-byte reads and 8 chains a
+// block in flight.
+template <typename T>
+__global__ __launch_bounds__(256) void sum_parts_kernel(int64_t n, int nparts, const T* __restrict__ part,
+                                                        T* __restrict__ out, int acc) {
+  __shared__ T red[8][32];
+  const int c = threadIdx.x & 31, grp = threadIdx.x >> 5;
+  for (int64_t i0 = (int64_t)blockIdx.x * 32; i0 < n; i0 += (int64_t)gridDim.x * 32) {
+    const int64_t idx = i0 + c;
+    T s = 0;
+    if (idx < n) {
+#pragma unroll 8
+      for (int p = grp; p < nparts; p += 8) s += part[(int64_t)p * n + idx];
+    }
+    red[grp][c] = s;
+    __syncthreads();
+    if (grp == 0 && idx < n) {
+#pragma unroll
+      for (int k = 1; k < 8; ++k) s += red[k][c];
+      put(out + idx, s, acc);
+    }
+    __syncthreads();
+  }
+}
+unsigned sum_parts_grid(int64_t n) { return (unsigned)std::min<int64_t>((n + 31) / 32, 4096); }
+
+// ---------------------------------------------------------------- channel mix (MFMA), fp64
+// Used for double, whose operands are twice as large; the fp32 forms are further down.
 // Rows are the (b, k) pairs R = b*K + k.  A wave takes two 16-row tiles and eight 16-column tiles; lane
 // (r, q) of an MFMA supplies A[r][4q..4q+3] and B[4q..4q+3][r] for a 16-deep K step and ends with
 // D[4q + j][r] in result register j (common.h).
@@ -283,9 +385,6 @@ __global__ __launch_bounds__(256) void mix_kernel(Dims d, const T* __restrict__ 
                                                   T* __restrict__ out, int acc) {
   using M = Mma<T>;
   using V = typename M::V;
-  // fp32 requests the next K step's operands before the current products (two register sets); fp64,
-  // whose operand sets are twice as large, works one step at a time
-  constexpr bool PF = sizeof(T) == 4;
   __shared__ T rs[128];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, q = lane >> 4;
@@ -351,27 +450,11 @@ __global__ __launch_bounds__(256) void mix_kernel(Dims d, const T* __restrict__ 
         for (int j = 0; j < 8; ++j) accm[t][j] = M::mma(a, bw[j], accm[t][j]);
       }
     };
-    if constexpr (PF) {
-      V a0[2], b0[8], a1[2], b1[8];
-      T g0[2], g1[2];
-      if (nst > 0) load(0, a0, g0, b0);
-      for (int st = 0; st < nst; st += 2) {
-        if (st + 1 < nst) load(st + 1, a1, g1, b1);
-        __builtin_amdgcn_sched_barrier(0);
-        mma(a0, g0, b0);
-        if (st + 1 < nst) {
-          if (st + 2 < nst) load(st + 2, a0, g0, b0);
-          __builtin_amdgcn_sched_barrier(0);
-          mma(a1, g1, b1);
-        }
-      }
-    } else {
-      for (int st = 0; st < nst; ++st) {
-        V a0[2], b0[8];
-        T g0[2];
-        load(st, a0, g0, b0);
-        mma(a0, g0, b0);
-      }
+    for (int st = 0; st < nst; ++st) {
+      V a0[2], b0[8];
+      T g0[2];
+      load(st, a0, g0, b0);
+      mma(a0, g0, b0);
     }
 #pragma unroll
     for (int t = 0; t < 2; ++t)
@@ -567,6 +650,353 @@ __global__ __launch_bounds__(256) void mix_tw_kernel(Dims d, const T* __restrict
     }
 }
 
+// ---------------------------------------------------------------- channel mix, fp32
+// The fp32 forms bound by the fp32 matrix rate (157 TFLOP/s): a block of four waves takes 128 rows x 128
+// columns, wave w the rows 32w .. 32w+31.  The column operand (weights, [column][contraction]) is common to the
+// four waves and goes through LDS 32 contraction steps at a time, rows padded to 36 floats (conflict-free
+// 16-byte reads); the next slice and the wave's own rows are requested a slice (4096 MFMA cycles) ahead.
+// 60,011 elements, K 7, 128 x 128 channels (13.8 GFLOP, y and out 0.43 GB): forward
+// 279 -> 262 us, gate gradient 485 -> 270, input gradient 309 -> 170 (81 TFLOP/s), weight gradient 333 + 515 for
+// its sum -> 252 + 9; every wave read the weights from L2 itself before.
+constexpr int KS = 32;          // contraction steps per slice
+constexpr int WPAD = KS + 4;
+constexpr int OPAD = 132;       // row stride of an output slice [32 columns][128 rows]; 32 * OPAD <= 128 * WPAD
+
+// The block's share of a weight slice in flight: 128 columns x 32 steps, four 16-byte pieces a thread.
+struct WSlice {
+  f4 v[4];
+  __device__ __forceinline__ void load(const float* __restrict__ w, int ncol, int nk, int c0, int k0) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const int c = c0 + (threadIdx.x >> 3) + 32 * s, k = k0 + 4 * (threadIdx.x & 7);
+      const bool ok = c < ncol && k < nk;
+      v[s] = ld4(w + (ok ? (int64_t)c * nk + k : 0));
+      if (!ok) v[s] = f4{0.f, 0.f, 0.f, 0.f};
+    }
+  }
+  __device__ __forceinline__ void store(float* ws) const {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) st4(ws + ((threadIdx.x >> 3) + 32 * s) * WPAD + 4 * (threadIdx.x & 7), v[s]);
+  }
+};
+
+// The products of one slice: a[h][t] holds the contraction steps 16h + 4q .. + 3 of row tile t.
+__device__ __forceinline__ void mma_slice(const f4 (&a)[2][2], const float* ws, int r, int q, f4 (&accm)[2][8]) {
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const f4 b = ld4(ws + (16 * j + r) * WPAD + 16 * h + 4 * q);
+#pragma unroll
+      for (int t = 0; t < 2; ++t) accm[t][j] = mfma_k16(a[h][t], b, accm[t][j]);
+    }
+}
+
+// out[b][o][k] (+)= sum_p g[b][p] sum_i y[b][p][k][i] W[p][o][i]; grid: 128 rows x 128 columns o.
+// TG: grad_g[b][p] (+)= sum_{k,o} go[b][o][k] sum_i y[b][p][k][i] W[p][o][i]; grid: 128/K whole elements x
+// paths, every column by the same block.
+template <bool TG>
+__global__ __launch_bounds__(256, 3) void mix32_kernel(Dims d, const float* __restrict__ y, const float* __restrict__ W,
+                                                       const float* __restrict__ g, const float* __restrict__ go,
+                                                       float* __restrict__ out, int acc) {
+  __shared__ float ws[128 * WPAD];
+  __shared__ float rs[128];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, q = lane >> 4;
+  const int K = d.K, P = d.P, I = d.I, O = d.O;
+  const uint32_t R = (uint32_t)(d.B * K);   // below 2^31 (checked): 32-bit row arithmetic, a 64-bit division by K
+  const int BB = 128 / K;                   // for each of a lane's rows took a third of the kernel
+  const uint32_t bb0 = blockIdx.x * BB;
+  const uint32_t rbeg = TG ? bb0 * K : blockIdx.x * 128;
+  const uint32_t rend = TG ? std::min((bb0 + BB) * (uint32_t)K, R) : std::min(rbeg + 128, R);
+  int64_t yb[2], rb[2];   // the lane's rows: offset of y at path 0, element
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const uint32_t row = rbeg + wave * 32 + 16 * t + r;
+    const uint32_t rr = row < rend ? row : rbeg;
+    rb[t] = rr / (uint32_t)K;
+    yb[t] = (rb[t] * P * K + (rr - (uint32_t)rb[t] * K)) * I;
+  }
+  const int ns = (I + KS - 1) / KS;
+  const int pb = TG ? (int)blockIdx.y : 0, pe = TG ? pb + 1 : P;
+  const int ob = TG ? 0 : (int)blockIdx.y * 128, oe = TG ? O : std::min(O, ob + 128);
+  float rowsum[2][4];
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) rowsum[t][j] = 0.f;
+  for (int o0 = ob; o0 < oe; o0 += 128) {
+    f4 accm[2][8];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) accm[t][j] = f4{0.f, 0.f, 0.f, 0.f};
+    // the slices of every path in order: position (p, s)
+    WSlice w;
+    f4 an[2][2];
+    float gn[2];
+    auto request = [&](int p, int s) {
+      w.load(W + (int64_t)p * O * I, O, I, o0, s * KS);
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        gn[t] = TG ? 1.f : g[rb[t] * P + p];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int i = s * KS + 16 * h + 4 * q;
+          an[h][t] = ld4(y + yb[t] + (int64_t)p * K * I + (i < I ? i : 0));
+        }
+      }
+    };
+    request(pb, 0);
+    int p = pb, s = 0;
+    while (p < pe) {
+      f4 a[2][2];
+      __syncthreads();   // the previous slice is read
+      w.store(ws);
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          a[h][t] = an[h][t] * gn[t];
+          if (s * KS + 16 * h + 4 * q >= I) a[h][t] = f4{0.f, 0.f, 0.f, 0.f};
+        }
+      int p1 = p, s1 = s + 1;
+      if (s1 == ns) { s1 = 0; ++p1; }
+      if (p1 < pe) request(p1, s1);
+      __syncthreads();
+      mma_slice(a, ws, r, q, accm);
+      p = p1;
+      s = s1;
+    }
+    if constexpr (TG) {
+      // loads at clamped addresses, so that they are all in flight together
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) {
+          const uint32_t row = std::min<uint32_t>(rbeg + wave * 32 + 16 * t + 4 * q + jj, rend - 1);
+          const uint32_t b = row / (uint32_t)K;
+          const float* gp = go + (int64_t)b * O * K + (row - b * K);
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            const int o = o0 + 16 * j + r;
+            const float gv = gp[(int64_t)std::min(o, O - 1) * K];
+            rowsum[t][jj] += o < O ? accm[t][j][jj] * gv : 0.f;
+          }
+        }
+    } else {
+      // out[b][o][k] holds an element's rows side by side: a store per register would write 4 bytes every 4K.
+      // 32 columns at a time pass through LDS, [column][row], and leave in runs of 32 K floats an element.
+      const uint32_t nrow = rend - rbeg, b0 = rbeg / (uint32_t)K, nb = (rend - 1) / (uint32_t)K - b0 + 1;
+#pragma unroll
+      for (int sl = 0; sl < 4; ++sl) {
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int jh = 0; jh < 2; ++jh)
+            st4(ws + (16 * jh + r) * OPAD + wave * 32 + 16 * t + 4 * q, accm[t][2 * sl + jh]);
+        __syncthreads();
+        const int oc = std::min(32, O - o0 - 32 * sl);   // columns of the slice
+        if (oc > 0) {
+          const uint32_t run = (uint32_t)oc * K;
+          for (uint32_t idx = threadIdx.x; idx < nb * run; idx += 256) {
+            const uint32_t bi = idx / run, rem = idx - bi * run, c = rem / (uint32_t)K, k = rem - c * K;
+            const int32_t lr = (int32_t)((b0 + bi) * K + k - rbeg);
+            if (lr >= 0 && lr < (int32_t)nrow)
+              put(out + ((int64_t)(b0 + bi) * O + o0 + 32 * sl) * K + rem, ws[c * OPAD + lr], acc);
+          }
+        }
+      }
+    }
+  }
+  if constexpr (TG) {
+    // row sums over the 16 column lanes, then over the K rows of each batch element
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int jj = 0; jj < 4; ++jj) {
+        float v = rowsum[t][jj];
+#pragma unroll
+        for (int off = 1; off < 16; off <<= 1) v += __shfl_xor(v, off, 64);
+        if (r == 0) rs[wave * 32 + 16 * t + 4 * q + jj] = v;
+      }
+    __syncthreads();
+    if (threadIdx.x < BB) {
+      const int64_t b = (int64_t)bb0 + threadIdx.x;
+      if (b < d.B) {
+        float v = 0.f;
+        for (int k = 0; k < K; ++k) v += rs[threadIdx.x * K + k];
+        put(out + b * P + pb, v, acc);
+      }
+    }
+  }
+}
+
+// grad_y[b][p][k][i] (+)= g[b][p] sum_o go[b][o][k] W[p][o][i]; grid: 128 rows x (path, 128 columns i), column
+// operand Wt[p][i][o].  Column 8r + j of the block is column r of tile j, so that a lane stores 8 channels in
+// a row.
+__global__ __launch_bounds__(256, 3) void mix32_ty_kernel(Dims d, const float* __restrict__ go,
+                                                          const float* __restrict__ Wt, const float* __restrict__ g,
+                                                          float* __restrict__ gy, int acc) {
+  __shared__ float ws[128 * WPAD];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, q = lane >> 4;
+  const int K = d.K, P = d.P, I = d.I, O = d.O;
+  const uint32_t R = (uint32_t)(d.B * K);
+  const int nib = (I + 127) / 128;
+  const int p = (int)blockIdx.y / nib, i0 = ((int)blockIdx.y % nib) * 128;
+  const uint32_t rbeg = blockIdx.x * 128;
+  int64_t gb[2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const uint32_t row = rbeg + wave * 32 + 16 * t + r;
+    const uint32_t rr = row < R ? row : 0, b = rr / (uint32_t)K;
+    gb[t] = (int64_t)b * O * K + (rr - b * K);
+  }
+  f4 accm[2][8];
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) accm[t][j] = f4{0.f, 0.f, 0.f, 0.f};
+  WSlice w;
+  f4 an[2][2];
+  auto request = [&](int k0) {
+    w.load(Wt + (int64_t)p * I * O, I, O, i0, k0);
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int o = k0 + 16 * h + 4 * q;
+        const float* gp = go + gb[t] + (int64_t)(o < O ? o : 0) * K;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) an[h][t][u] = gp[(int64_t)u * K];
+      }
+  };
+  request(0);
+  for (int k0 = 0; k0 < O; k0 += KS) {
+    f4 a[2][2];
+    __syncthreads();
+    // columns re-ordered on the way into LDS: row 16j + r of the slice is column 8r + j
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const int c = (threadIdx.x >> 3) + 32 * s;
+      st4(ws + (16 * (c & 7) + (c >> 3)) * WPAD + 4 * (threadIdx.x & 7), w.v[s]);
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        a[h][t] = an[h][t];
+        if (k0 + 16 * h + 4 * q >= O) a[h][t] = f4{0.f, 0.f, 0.f, 0.f};
+      }
+    if (k0 + KS < O) request(k0 + KS);
+    __syncthreads();
+    mma_slice(a, ws, r, q, accm);
+  }
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int jj = 0; jj < 4; ++jj) {
+      const uint32_t row = rbeg + wave * 32 + 16 * t + 4 * q + jj;
+      if (row >= R) continue;
+      const uint32_t b = row / (uint32_t)K;
+      const float gate = g[(int64_t)b * P + p];
+      float* o = gy + (((int64_t)b * P + p) * K + (row - b * K)) * I + i0 + 8 * r;
+#pragma unroll
+      for (int hh = 0; hh < 2; ++hh)
+        if (i0 + 8 * r + 4 * hh < I) {   // I % 4 == 0
+          f4 v = {accm[t][4 * hh][jj], accm[t][4 * hh + 1][jj], accm[t][4 * hh + 2][jj], accm[t][4 * hh + 3][jj]};
+          v = v * gate;
+          if (acc) v = ld4(o + 4 * hh) + v;
+          st4(o + 4 * hh, v);
+        }
+    }
+}
+
+// Partial sums of grad_W[p][o][i] = sum_{(b,k)} g[b][p] go[b][o][k] y[b][p][k][i] over a range of rows.  Block
+// (split, path, 128 x 128 tile); both operands go through LDS 32 rows at a time (each read from memory once a
+// block instead of once a wave), the next rows in flight meanwhile; wave w takes a 64 x 64 quarter.
+constexpr int TPAD = 128 + 16;   // row stride of the staged rows: the four rows of an MFMA step on distinct banks
+__global__ __launch_bounds__(256, 3) void mix32_tw_kernel(Dims d, const float* __restrict__ go,
+                                                          const float* __restrict__ y, const float* __restrict__ g,
+                                                          int64_t rows_per_split, float* __restrict__ part) {
+  __shared__ float gs[KS * TPAD];
+  __shared__ float ys[KS * TPAD];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, q = lane >> 4;
+  const int K = d.K, P = d.P, I = d.I, O = d.O;
+  const uint32_t R = (uint32_t)(d.B * K);
+  const int s = blockIdx.x, p = blockIdx.y;
+  const int nib = (I + 127) / 128;
+  const int o0 = ((int)blockIdx.z / nib) * 128, i0 = ((int)blockIdx.z % nib) * 128;
+  const uint32_t r0 = (uint32_t)(s * rows_per_split), r1 = (uint32_t)std::min<int64_t>(R, r0 + rows_per_split);
+  const int wo = 64 * (wave >> 1), wi = 64 * (wave & 1);
+  f4 accm[4][4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) accm[t][j] = f4{0.f, 0.f, 0.f, 0.f};
+  f4 yn[4];
+  float gn[16];
+  const int ycol = i0 + 4 * (threadIdx.x & 31);
+  const int ocol = o0 + (threadIdx.x & 127), orow = __builtin_amdgcn_readfirstlane(threadIdx.x >> 7) * 16;
+  auto request = [&](uint32_t rr) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {   // y: row (tid / 32) + 8u, 4 channels
+      const uint32_t row = rr + (threadIdx.x >> 5) + 8 * u;
+      const bool ok = row < r1 && ycol < I;
+      const uint32_t rw = ok ? row : r0, b = rw / (uint32_t)K;
+      yn[u] = ld4(y + (((int64_t)b * P + p) * K + (rw - b * K)) * I + (ok ? ycol : 0));
+      if (!ok) yn[u] = f4{0.f, 0.f, 0.f, 0.f};
+    }
+    // go: 16 rows (the same for the wave) of one column; the element and row in it advance without divisions
+    uint32_t b = std::min(rr + orow, r1 - 1) / (uint32_t)K, k = std::min(rr + orow, r1 - 1) - b * K;
+    const float* gc = go + (int64_t)(ocol < O ? ocol : 0) * K;
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+      const float v = gc[(int64_t)b * O * K + k] * g[(int64_t)b * P + p];
+      gn[u] = rr + orow + u < r1 && ocol < O ? v : 0.f;
+      if (rr + orow + u + 1 < r1 && ++k == (uint32_t)K) { k = 0; ++b; }
+    }
+  };
+  request(r0);
+  for (uint32_t rr = r0; rr < r1; rr += KS) {
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 4; ++u) st4(ys + ((threadIdx.x >> 5) + 8 * u) * TPAD + 4 * (threadIdx.x & 31), yn[u]);
+#pragma unroll
+    for (int u = 0; u < 16; ++u) gs[(orow + u) * TPAD + (threadIdx.x & 127)] = gn[u];
+    if (rr + KS < r1) request(rr + KS);
+    __syncthreads();
+#pragma unroll
+    for (int k4 = 0; k4 < KS; k4 += 4) {
+      float a[4], b[4];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) a[t] = gs[(k4 + q) * TPAD + wo + 16 * t + r];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) b[j] = ys[(k4 + q) * TPAD + wi + 16 * j + r];
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) accm[t][j] = mfma16x16x4(a[t], b[j], accm[t][j]);
+    }
+  }
+  float* ps = part + ((int64_t)s * P + p) * O * I;
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int jj = 0; jj < 4; ++jj) {
+      const int o = o0 + wo + 16 * t + 4 * q + jj;
+      if (o >= O) continue;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int i = i0 + wi + 16 * j + r;
+        if (i < I) ps[(int64_t)o * I + i] = accm[t][j][jj];
+      }
+    }
+}
+
 // ---------------------------------------------------------------- host side
 int check_dims(const Dims& d, bool proj) {
   FSC_CHECK_ARG(d.B >= 0 && d.I > 0 && d.P > 0 && d.K > 0, "bucket op: sizes must be positive");
@@ -587,6 +1017,31 @@ size_t proj_t_lds(const Dims& d, bool do_u, size_t elem) {
   const int PK = d.P * d.K, MN = d.m1 * d.m2;
   const size_t main = (size_t)(MN * PK + 4 * (IC * d.m1 + IC * (PK + 1) + d.m1 * PK)) * elem;
   return do_u ? std::max(main, (size_t)4 * MN * PK * elem) : main;
+}
+
+bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
+template <typename T>
+size_t project_tv_lds(const Dims& d) { return (size_t)d.m2 * 256 * ((d.P * d.K + 15) / 16) * sizeof(T); }
+// whole aligned 4-vectors of channels, and the padded factor within 64 KB (only fp64 at m2 9, PK > 48 exceeds it)
+template <typename T>
+bool project_tv_ok(const Dims& d, const T* gy) {
+  return d.I % 4 == 0 && aligned16(gy) && project_tv_lds<T>(d) <= 65536;
+}
+
+template <typename T>
+void launch_project_tv(const Dims& d, const T* gy, const T* a, const T* u, T* grad_v, int acc, hipStream_t st) {
+  const int nt = (d.P * d.K + 15) / 16;
+  const size_t lds = project_tv_lds<T>(d);
+  const unsigned grid = std::min(batch_grid(d.B), 2048u);   // resident at once: the factor is staged once a block
+  if (nt == 1)
+    project_tv_kernel<T, 1><<<grid, 256, lds, st>>>(d, gy, a, u, grad_v, acc);
+  else if (nt == 2)
+    project_tv_kernel<T, 2><<<grid, 256, lds, st>>>(d, gy, a, u, grad_v, acc);
+  else if (nt == 3)
+    project_tv_kernel<T, 3><<<grid, 256, lds, st>>>(d, gy, a, u, grad_v, acc);
+  else
+    project_tv_kernel<T, 4><<<grid, 256, lds, st>>>(d, gy, a, u, grad_v, acc);
 }
 
 // ---------------------------------------------------------------- entry points, for T = float and double
@@ -640,6 +1095,8 @@ int project_transpose_vu(int64_t B, int32_t I, int32_t m1, int32_t m2, int32_t P
     const size_t lds = proj_t_lds(d, grad_u != nullptr, sizeof(T));
     if (grad_v && grad_u)
       project_t_kernel<T, true, true><<<grid, 256, lds, st>>>(d, grad_y, a, v, u, grad_v, accumulate, workspace);
+    else if (grad_v && project_tv_ok<T>(d, grad_y))
+      launch_project_tv<T>(d, grad_y, a, u, grad_v, accumulate, st);
     else if (grad_v)
       project_t_kernel<T, true, false><<<grid, 256, lds, st>>>(d, grad_y, a, v, u, grad_v, accumulate, nullptr);
     else
@@ -648,8 +1105,7 @@ int project_transpose_vu(int64_t B, int32_t I, int32_t m1, int32_t m2, int32_t P
   }
   if (grad_u) {
     // (no elements: a sum over zero parts, which writes zeros or leaves an accumulated output unchanged)
-    sum_parts_kernel<T><<<(unsigned)std::min<int64_t>((mnpk + 255) / 256, 1024), 256, 0, st>>>(
-        mnpk, B > 0 ? (int)grid : 0, workspace, grad_u, accumulate);
+    sum_parts_kernel<T><<<sum_parts_grid(mnpk), 256, 0, st>>>(mnpk, B > 0 ? (int)grid : 0, workspace, grad_u, accumulate);
     if (check_launch("bucket project_transpose_u reduce")) return 2;
   }
   return 0;
@@ -662,7 +1118,10 @@ int mix(int64_t B, int32_t P, int32_t K, int32_t I, int32_t O, const T* y, const
   if (check_dims(d, false)) return 1;
   if (B == 0) return 0;
   const dim3 grid((unsigned)((B * K + 127) / 128), (unsigned)((O + 127) / 128));
-  mix_kernel<T, false><<<grid, 256, 0, st>>>(d, y, w, gates, nullptr, out, accumulate);
+  if constexpr (std::is_same_v<T, float>)
+    mix32_kernel<false><<<grid, 256, 0, st>>>(d, y, w, gates, nullptr, out, accumulate);
+  else
+    mix_kernel<T, false><<<grid, 256, 0, st>>>(d, y, w, gates, nullptr, out, accumulate);
   return check_launch("bucket mix") ? 2 : 0;
 }
 
@@ -674,14 +1133,17 @@ int mix_transpose_g(int64_t B, int32_t P, int32_t K, int32_t I, int32_t O, const
   if (B == 0) return 0;
   const int BB = 128 / K;
   const dim3 grid((unsigned)((B + BB - 1) / BB), (unsigned)P);
-  mix_kernel<T, true><<<grid, 256, 0, st>>>(d, y, w, nullptr, grad_out, grad_g, accumulate);
+  if constexpr (std::is_same_v<T, float>)
+    mix32_kernel<true><<<grid, 256, 0, st>>>(d, y, w, nullptr, grad_out, grad_g, accumulate);
+  else
+    mix_kernel<T, true><<<grid, 256, 0, st>>>(d, y, w, nullptr, grad_out, grad_g, accumulate);
   return check_launch("bucket mix_transpose_g") ? 2 : 0;
 }
 
 int64_t mix_tw_splits(int64_t B, int32_t P, int32_t K, int32_t I, int32_t O, int64_t* rows_per_split) {
   const int64_t R = std::max<int64_t>(B * K, 1);
   const int64_t tiles = (int64_t)P * ((O + 127) / 128) * ((I + 127) / 128);
-  const int64_t want = std::max<int64_t>(1, 2048 / tiles);
+  const int64_t want = std::max<int64_t>(1, 768 / tiles);   // three blocks a CU
   int64_t rps = std::max<int64_t>(256, (R + want - 1) / want);
   rps = (rps + 15) / 16 * 16;
   *rows_per_split = rps;
@@ -707,7 +1169,10 @@ int mix_transpose_y(int64_t B, int32_t P, int32_t K, int32_t I, int32_t O, const
   transpose_w_kernel<T><<<(unsigned)std::min<int64_t>((nw + 255) / 256, 4096), 256, 0, st>>>(P, O, I, w, workspace);
   if (check_launch("bucket transpose_w")) return 2;
   const dim3 grid((unsigned)((B * K + 127) / 128), (unsigned)(P * ((I + 127) / 128)));
-  mix_ty_kernel<T><<<grid, 256, 0, st>>>(d, grad_out, workspace, gates, grad_y, accumulate);
+  if constexpr (std::is_same_v<T, float>)
+    mix32_ty_kernel<<<grid, 256, 0, st>>>(d, grad_out, workspace, gates, grad_y, accumulate);
+  else
+    mix_ty_kernel<T><<<grid, 256, 0, st>>>(d, grad_out, workspace, gates, grad_y, accumulate);
   return check_launch("bucket mix_transpose_y") ? 2 : 0;
 }
 
@@ -718,17 +1183,18 @@ int mix_transpose_w(int64_t B, int32_t P, int32_t K, int32_t I, int32_t O, const
   if (check_dims(d, false)) return 1;
   const int64_t nw = (int64_t)P * O * I;
   if (B == 0) {   // a sum over zero parts
-    sum_parts_kernel<T><<<(unsigned)std::min<int64_t>((nw + 255) / 256, 4096), 256, 0, st>>>(nw, 0, workspace, grad_w,
-                                                                                           accumulate);
+    sum_parts_kernel<T><<<sum_parts_grid(nw), 256, 0, st>>>(nw, 0, workspace, grad_w, accumulate);
     return check_launch("bucket mix_transpose_w") ? 2 : 0;
   }
   int64_t rps;
   const int64_t ns = mix_tw_splits(B, P, K, I, O, &rps);
   const dim3 grid((unsigned)ns, (unsigned)P, (unsigned)(((O + 127) / 128) * ((I + 127) / 128)));
-  mix_tw_kernel<T><<<grid, 256, 0, st>>>(d, grad_out, y, gates, rps, workspace);
+  if constexpr (std::is_same_v<T, float>)
+    mix32_tw_kernel<<<grid, 256, 0, st>>>(d, grad_out, y, gates, rps, workspace);
+  else
+    mix_tw_kernel<T><<<grid, 256, 0, st>>>(d, grad_out, y, gates, rps, workspace);
   if (check_launch("bucket mix_transpose_w")) return 2;
-  sum_parts_kernel<T><<<(unsigned)std::min<int64_t>((nw + 255) / 256, 4096), 256, 0, st>>>(nw, (int)ns, workspace,
-                                                                                         grad_w, accumulate);
+  sum_parts_kernel<T><<<sum_parts_grid(nw), 256, 0, st>>>(nw, (int)ns, workspace, grad_w, accumulate);
   return check_launch("bucket mix_transpose_w reduce") ? 2 : 0;
 }
 

@@ -93,6 +93,27 @@ def test_mix_ops(case, dt):
     assert max(errs.values()) < TOL, errs
 
 
+# tile edges: rows straddling elements (K 3, 5, 7, 9 with 128-row blocks), channels past one 128-column block and
+# past a 32-step slice, more row splits than one; factor columns P*K at each 16-wide tile count, channel tails,
+# m2 above and at 8
+@pytest.mark.parametrize("case", [(43, 1, 3, 132, 132), (129, 1, 1, 32, 4), (19, 3, 7, 100, 260), (128, 2, 5, 28, 128),
+                                  (3000, 1, 9, 64, 36), (1, 1, 128, 4, 4)])
+def test_mix_ops_at_tile_edges(case):
+    test_mix_ops(case, torch.float32)
+
+
+@pytest.mark.parametrize("case", [(5, 16, 9, 9, 1, 16), (9, 20, 3, 8, 1, 17), (7, 12, 9, 9, 4, 8), (6, 4, 1, 9, 3, 11),
+                                  (3, 36, 5, 1, 7, 7), (8193, 8, 3, 5, 1, 64), (11, 18, 3, 3, 2, 3)])
+def test_direction_gradient_at_tile_edges(case):
+    B, I, m1, m2, P, K = case
+    s = sum(case)
+    a, b, u = rnd(B, I, m1, seed=s), rnd(B, 1, m2, seed=s + 1), rnd(m1 * m2, P * K, seed=s + 2)
+    gy = rnd(B, P, K, I, seed=s + 3)
+    for dt, tol in TOLS.items():
+        got = ext().project_bucket_transpose_b(gpu(gy, dt), gpu(a, dt), gpu(u, dt))
+        assert rel(got, BR.project_transpose(gy, a, b, u)[1]) < tol
+
+
 @DTYPES
 def test_bucketed_tp_forward_and_double_backward(dt):
     E = ext()
