@@ -1062,8 +1062,22 @@ __global__ __launch_bounds__(256) void grad_absmax_kernel(const float* __restric
 // 888 us with fp32 products, 741 us here).  The bias column sums the two
 // planes over the edges on the VALU.  A lane's dh B operand is 8 consecutive chunk columns of one k (S
 // loads at a fixed stride, as in the fp32 kernel); a lane's dS B operand is 8 consecutive edges of one
-// column (eight 2-byte LDS reads per plane).  K = 144 is four 32-deep steps and a 16-deep one.
+// column, read by two transposing LDS reads (lds_column8; eight 2-byte reads a plane made the LDS pipe the
+// bound: 10,000 nodes, C 64, 1893 -> 1707 us; 4,099 nodes bf16, 741 -> 651).  K = 144 is four 32-deep steps and a 16-deep one.
 typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+typedef float f2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ f2 ld2(const float* p) { return *reinterpret_cast<const f2*>(p); }
+
+// ds_read_b64_tr_b16: in each group of 16 lanes, lane i names four fp16 of row i/4, columns 4(i%4)..+3 of a
+// 4 x 16 block and receives column i of its four rows (checked on gfx950).  Two reads: eight rows of a column.
+__device__ __forceinline__ h8 lds_column8(const _Float16* rows0, const _Float16* rows4) {
+  typedef short s4 __attribute__((__vector_size__(8)));
+  typedef __attribute__((address_space(3))) s4* lp;
+  const h4 a = __builtin_bit_cast(h4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lp)(const_cast<_Float16*>(rows0))));
+  const h4 b = __builtin_bit_cast(h4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lp)(const_cast<_Float16*>(rows4))));
+  return h8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+}
 constexpr int DPS = 144;   // fp16 row stride of dP in LDS (144 columns, 288 bytes: 16-byte aligned rows)
 
 template <int C, bool BF16S>
@@ -1113,8 +1127,8 @@ __global__ __launch_bounds__(256, 4) void edge_message_grad_h16_kernel(
   const uint32_t svoff = (uint32_t)((q * COLS + 16 * wave + r) * SB);
   const uint32_t svoff_t = (uint32_t)(((q >> 1) * COLS + 4 * (q & 1) * KH + 16 * wave + r) * SB);
   const uint32_t dvoff = (uint32_t)(((r >> 3) * COLS + (r & 7) * KH + 16 * wave + 4 * q) * 4);
-  const int cl = threadIdx.x & (CC - 1);   // dP builder: channel within the chunk
-  const int eb = threadIdx.x / CC;         // dP builder: edges eb, eb + 32
+  const int cl = 2 * (threadIdx.x & 3);    // dP builder: channels cl, cl + 1 of the chunk
+  const int eb = threadIdx.x >> 2;         // dP builder: edge
 
   if (end == beg) {   // no out-edges: dS of this node is zero (block-uniform branch; part 0 writes it)
     if (part == 0)
@@ -1176,21 +1190,18 @@ __global__ __launch_bounds__(256, 4) void edge_message_grad_h16_kernel(
 #pragma unroll
     for (int et = 0; et < 4; ++et) dacc[et] = f4{0.f, 0.f, 0.f, 0.f};
 
-    float gN[2][NCOMP], pN[2][5], sv[36];
+    f2 gN[NCOMP], pN[5];
+    float sv[36];
     auto load_g = [&](int ch) {
+      const float* gp = Gt + ((int64_t)ch * n_nodes + dsts[eb]) * (NCOMP * CC) + cl;
 #pragma unroll
-      for (int hh = 0; hh < 2; ++hh) {
-        const int e = eb + 32 * hh;
-        const float* gp = Gt + ((int64_t)ch * n_nodes + dsts[e]) * (NCOMP * CC) + cl;
-#pragma unroll
-        for (int i = 0; i < NCOMP; ++i) gN[hh][i] = gp[i * CC];
-        const float* pp = P + (int64_t)eids[e] * NCOL + ch * 40 + cl;   // p_col of positions 0..4
-        pN[hh][0] = pp[pos_of_slot(1) * CC];
-        pN[hh][1] = pp[pos_of_slot(2) * CC];
-        pN[hh][2] = pp[pos_of_slot(6) * CC];
-        pN[hh][3] = pp[pos_of_slot(7) * CC];
-        pN[hh][4] = pp[pos_of_slot(8) * CC];
-      }
+      for (int i = 0; i < NCOMP; ++i) gN[i] = ld2(gp + i * CC);
+      const float* pp = P + (int64_t)eids[eb] * NCOL + ch * 40 + cl;   // p_col of positions 0..4
+      pN[0] = ld2(pp + pos_of_slot(1) * CC);
+      pN[1] = ld2(pp + pos_of_slot(2) * CC);
+      pN[2] = ld2(pp + pos_of_slot(6) * CC);
+      pN[3] = ld2(pp + pos_of_slot(7) * CC);
+      pN[4] = ld2(pp + pos_of_slot(8) * CC);
     };
     auto ld_s = [&](uint32_t vo, uint32_t so) {
       return BF16S ? buffer_ld1_bf16(srs, vo, so) : buffer_ld1(srs, vo, so);
@@ -1209,53 +1220,48 @@ __global__ __launch_bounds__(256, 4) void edge_message_grad_h16_kernel(
     for (int ch = ch0; ch < ch1; ++ch) {
       const int c0 = ch * CC;
       load_g(ch);
-      // ---- dP for edges eb, eb+32 and channel c0+cl (scaled by s_e, split into the two planes);
-      //      direction-gradient partials in fp32
+      // ---- dP for edge eb and channels c0+cl, c0+cl+1 (scaled by s_e, split into the two planes, the two
+      //      channels' parts stored as one word); direction-gradient partials in fp32
+      {
+        const float sc = (eb < cnt) ? scale : 0.f, se = esc[eb];
+        const float nn[3] = {ns[eb][0], ns[eb][1], ns[eb][2]};
+        float t[3] = {0.f, 0.f, 0.f};
+        auto put = [&](int slot, f2 v) {
+          const f2 x = v * se;
+          const h2 xh = {(_Float16)x.x, (_Float16)x.y};
+          const h2 xl = {(_Float16)(x.x - (float)xh.x), (_Float16)(x.y - (float)xh.y)};
+          *reinterpret_cast<h2*>(&dpl[0][eb][slot * CC + cl]) = xh;
+          *reinterpret_cast<h2*>(&dpl[1][eb][slot * CC + cl]) = xl;
+        };
+        f2 g[NCOMP];
 #pragma unroll
-      for (int hh = 0; hh < 2; ++hh) {
-        const int e = eb + 32 * hh;
-        float v[NSLOT];
-        float t[3];
-        float g[NCOMP];
-        const float sc = (e < cnt) ? scale : 0.f;
-#pragma unroll
-        for (int i = 0; i < NCOMP; ++i) g[i] = gN[hh][i] * sc;
-        const float nn[3] = {ns[e][0], ns[e][1], ns[e][2]};
-        const float p1 = pN[hh][0], p2 = pN[hh][1];
-        const float p4[3] = {pN[hh][2], pN[hh][3], pN[hh][4]};
-        v[0] = g[0];
-        v[1] = g[1] * nn[0] + g[2] * nn[1] + g[3] * nn[2];
-        float nqn = 0.f;
+        for (int i = 0; i < NCOMP; ++i) g[i] = gN[i] * sc;
+        put(0, g[0]);
+        put(1, g[1] * nn[0] + g[2] * nn[1] + g[3] * nn[2]);
+        f2 nqn = {0.f, 0.f};
 #pragma unroll
         for (int i = 0; i < 3; ++i) {
-          float row = 0.f, colv = 0.f, p4t = 0.f;
+          f2 row = {0.f, 0.f}, colv = {0.f, 0.f}, p4t = {0.f, 0.f};
 #pragma unroll
           for (int j = 0; j < 3; ++j) {
             row += g[4 + 3 * i + j] * nn[j];
             colv += g[4 + 3 * j + i] * nn[j];
-            p4t += g[4 + 3 * j + i] * p4[j];
+            p4t += g[4 + 3 * j + i] * pN[2 + j];
           }
-          v[3 + i] = g[1 + i];
-          v[6 + i] = row;
+          put(3 + i, g[1 + i]);
+          put(6 + i, row);
           nqn += row * nn[i];
-          t[i] = g[1 + i] * p1 + p2 * (row + colv) + p4t;
+          const f2 ti = g[1 + i] * pN[0] + pN[1] * (row + colv) + p4t;
+          t[i] = ti.x + ti.y;
         }
-        v[2] = nqn;
+        put(2, nqn);
 #pragma unroll
-        for (int i = 0; i < 9; ++i) v[9 + i] = g[4 + i];
-        const float se = esc[e];
+        for (int i = 0; i < 9; ++i) put(9 + i, g[4 + i]);
 #pragma unroll
-        for (int s4 = 0; s4 < NSLOT; ++s4) {
-          const float x = v[s4] * se;
-          const _Float16 xh = (_Float16)x;
-          dpl[0][e][s4 * CC + cl] = xh;
-          dpl[1][e][s4 * CC + cl] = (_Float16)(x - (float)xh);
-        }
+        for (int k = 0; k < 3; ++k) t[k] = group_sum(t[k], CC / 2);
+        if (cl == 0 && eb < cnt) {
 #pragma unroll
-        for (int k = 0; k < 3; ++k) t[k] = group_sum(t[k], CC);
-        if (cl == 0 && e < cnt) {
-#pragma unroll
-          for (int k = 0; k < 3; ++k) dnacc[e][k] += t[k];
+          for (int k = 0; k < 3; ++k) dnacc[eb][k] += t[k];
         }
       }
       // ---- dh B operand: the chunk's S values of column k = 16 w + r, scaled by their own power of two
@@ -1329,12 +1335,9 @@ __global__ __launch_bounds__(256, 4) void edge_message_grad_h16_kernel(
 #pragma unroll
             for (int u = 0; u < CTG; ++u) {
               const int ct = cg + u;
-              h8 xh, xl;
-#pragma unroll
-              for (int j = 0; j < 8; ++j) {
-                xh[j] = dpl[0][32 * s + 8 * q + j][16 * ct + r];
-                xl[j] = dpl[1][32 * s + 8 * q + j][16 * ct + r];
-              }
+              const int e0 = 32 * s + 8 * q + (r >> 2), col = 16 * ct + 4 * (r & 3);
+              const h8 xh = lds_column8(&dpl[0][e0][col], &dpl[0][e0 + 4][col]);
+              const h8 xl = lds_column8(&dpl[1][e0][col], &dpl[1][e0 + 4][col]);
               sacc[u] = mfma_x3(ah[s], al[s], xh, xl, sacc[u]);
             }
           }
