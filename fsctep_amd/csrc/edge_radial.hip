@@ -19,19 +19,12 @@ namespace radial {
 
 constexpr int HID = 64;     // hidden width of the radial MLP (fixed by the reference's fc)
 constexpr int NBMAX = 16;   // radial basis functions supported
-constexpr int RADW_RED = 16;   // block-reduction slots (at most 16 waves per block)
+constexpr int RADW_RED = 16;   // block-reduction slots (two maxima of at most 8 waves)
 
-// sin x and cos x for 0 <= x < 2^7: Cody-Waite reduction by pi/2 in two parts (the fma keeps
-// x - n*P1 to one rounding, and n*(pi/2 - P1 - P2) is below 2^-30 here), then the Taylor series on
-// [-pi/4, pi/4] to x^11 / x^12 (truncation below 1e-11) and the quadrant.  The basis argument is at
-// most nb*pi; the library sinf/cosf carry a large-argument path whose registers the radial MLP kernels
-// cannot spare.
-__device__ __forceinline__ void sincos_small(float x, float& s, float& c) {
-  constexpr float P1 = 1.57079637050628662109375f;       // pi/2 rounded to float
-  constexpr float P2 = -4.37113900018624283e-8f;         // pi/2 - P1
-  const float n = rintf(x * 0.636619772367581343f);      // x / (pi/2)
-  float t = fmaf(-n, P1, x);
-  t = fmaf(-n, P2, t);
+// sin and cos of t + n pi/2 for |t| <= pi/4 (and a little beyond): Taylor series to t^11 / t^12 (truncation below
+// 1e-11) and the quadrant.  The library sinf/cosf carry a large-argument path whose registers the radial MLP
+// kernels cannot spare.
+__device__ __forceinline__ void sincos_quadrant(float t, float n, float& s, float& c) {
   const float t2 = t * t;
   const float sp = t + t * t2 * (-1.f / 6.f + t2 * (1.f / 120.f + t2 * (-1.f / 5040.f + t2 * (1.f / 362880.f +
                                                                       t2 * (-1.f / 39916800.f)))));
@@ -40,6 +33,27 @@ __device__ __forceinline__ void sincos_small(float x, float& s, float& c) {
   const int qd = ((int)n) & 3;
   s = (qd == 0) ? sp : (qd == 1) ? cp : (qd == 2) ? -sp : -cp;
   c = (qd == 0) ? cp : (qd == 1) ? -sp : (qd == 2) ? -cp : sp;
+}
+
+// sin x and cos x for 0 <= x < 2^7: Cody-Waite reduction by pi/2 in two parts (the fma keeps x - n*P1 to one
+// rounding, and n*(pi/2 - P1 - P2) is below 2^-30 here).
+__device__ __forceinline__ void sincos_small(float x, float& s, float& c) {
+  constexpr float P1 = 1.57079637050628662109375f;       // pi/2 rounded to float
+  constexpr float P2 = -4.37113900018624283e-8f;         // pi/2 - P1
+  const float n = rintf(x * 0.636619772367581343f);      // x / (pi/2)
+  float t = fmaf(-n, P1, x);
+  t = fmaf(-n, P2, t);
+  sincos_quadrant(t, n, s, c);
+}
+
+// sin and cos of pi k (uh + ul), k <= 16: the half turns k uh = p + e exactly, p less its nearest multiple of 1/2
+// exactly, so the argument keeps its last bits (rounding k pi r / rc to float costs k pi 2^-25 of absolute error,
+// the largest part of the radial MLP's).
+__device__ __forceinline__ void sincos_pi(float k, float uh, float ul, float& s, float& c) {
+  const float p = k * uh;
+  const float e = fmaf(k, uh, -p) + k * ul;
+  const float n = rintf(2.f * p);
+  sincos_quadrant((fmaf(-0.5f, n, p) + e) * 3.14159265358979323846f, n, s, c);
 }
 
 // emb_k(r) and d emb_k / dr for k < nb, e3nn's soft_one_hot_linspace(r, 0, rc, nb, basis, cutoff=True)
@@ -54,11 +68,12 @@ __device__ __forceinline__ void basis_eval(float r, int k, int nb, float rc, int
   const float snb = sqrtf((float)nb);
   if (basis == 0 || basis == 2) {
     const float w = (float)(k + 1) * (3.14159265358979323846f / rc);
-    const bool inside = (r / rc < 1.f) && (r > 0.f);
+    const bool inside = (r < rc) && (r > 0.f);   // r < rc exactly where the rounded r / rc is below 1
     const float rr = inside ? r : 1.f;
     const float x = w * rr;
+    const float uh = rr / rc, ul = fmaf(-uh, rc, rr) / rc;   // r / rc to twice the precision
     float s, c;
-    sincos_small(x, s, c);
+    sincos_pi((float)(k + 1), uh, ul, s, c);
     if (basis == 2) {
       const float a = snb * rsqrtf(0.25f + 0.5f * (float)nb);
       f = inside ? a * s : 0.f;
@@ -97,8 +112,14 @@ __device__ __forceinline__ void basis_eval(float r, int k, int nb, float rc, int
   }
 }
 
-// logistic sigmoid with the hardware exp2 and reciprocal (relative error ~1e-7)
-__device__ __forceinline__ float sigm(float x) { return __fdividef(1.f, 1.f + __expf(-x)); }
+// logistic sigmoid with the hardware exp2 and reciprocal (1 ulp each).  The kernels are bound by their VALU
+// operations and take 32 (forward) or 48 (backward) of these a lane and tile: a division instead of the
+// reciprocal is 10 more operations (__fdividef compiles to the full division).  An overflowing exponential
+// gives 1/inf = 0.
+__device__ __forceinline__ float sigm(float x) { return __builtin_amdgcn_rcpf(1.f + __expf(-x)); }
+
+// 1/s of a power of two s = 2^k, |k| <= 126, by its exponent field
+__device__ __forceinline__ float pow2_inverse(float s) { return __uint_as_float(0x7F000000u - __float_as_uint(s)); }
 
 // One wave per 16-edge tile; lane (r, q) works for edge e0 + r.  The hidden units are laid
 // out as the MFMA output: lane (r, q) holds unit j = 16*jt + 4*q + i in register (jt, i), so
@@ -125,69 +146,121 @@ struct Smem {
   LayerH16 w2;                                      // W2 (forward product; recomputed in the backward)
   std::conditional_t<BWD, LayerH16, NoLayer> w2t;   // W2^T (backward)
   LayerH16 w4;                                      // W4 in the forward, W4^T in the backward
-  float b0[HID];
-  float b2[HID];
-  float b4[HID];
+  alignas(16) float b0[HID];
+  alignas(16) float b2[HID];
+  alignas(16) float b4[HID];
   float winv[3];                // 1/sw of w2, w2t, w4
   float red[RADW_RED];
 };
+
+// Row of basis function k in W0^T: the product's result register i of lane group q is row 4q + i, and the lane
+// holds the derivatives of the functions 4i + q.
+__host__ __device__ constexpr int w0t_row(int k) { return 4 * (k & 3) + (k >> 2); }
 
 // K slot of hidden unit u in a layer's planes
 __host__ __device__ constexpr int kslot(int u) {
   return 32 * (u >> 5) + 8 * ((u >> 2) & 3) + 4 * ((u >> 4) & 1) + (u & 3);
 }
 
-// Planes of M (64 rows o, 64 columns u): p[h/l][o][kslot(u)] = split of M[o][u] sw, sw from the block's max
-// |M|; returns 1/sw (all threads).  get(o, u) reads M.
-template <typename Get>
-__device__ float stage_h16(LayerH16& L, float* red, Get get) {
-  float mx = 0.f;
-  for (int i = threadIdx.x; i < HID * HID; i += blockDim.x) mx = fmaxf(mx, fabsf(get(i / HID, i % HID)));
-  for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
-  __syncthreads();   // red is free (a previous call's readers are done)
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
-  __syncthreads();
-  mx = 0.f;
-  for (int w = 0; w < (int)(blockDim.x >> 6); ++w) mx = fmaxf(mx, red[w]);
-  const float sw = pow2_scale(mx);
-  for (int i = threadIdx.x; i < HID * HID; i += blockDim.x) {
-    const int o = i / HID, u = i % HID;
-    const float v = get(o, u) * sw;
-    const _Float16 h = (_Float16)v;
-    L.p[0][o][kslot(u)] = h;
-    L.p[1][o][kslot(u)] = (_Float16)(v - (float)h);
-  }
-  return 1.f / sw;   // exact: a power of two
-}
+// Blocks of RAD_WAVES waves share one LDS copy of the weights; two blocks per CU give 4 waves per SIMD
+// (at most 128 VGPRs), enough to overlap the dependent layers of one 16-edge tile with other tiles.
+constexpr int RAD_WAVES = 8;
+constexpr int RAD_THREADS = 64 * RAD_WAVES;
 
+// The block's share of a 64 x 64 layer in registers: two runs of four values a thread (row run / 16, columns
+// 4 (run % 16) ..), zero for rows past nrow.
+struct WRegs {
+  float v[2][4];
+  __device__ __forceinline__ void load(const float* __restrict__ W, int nrow) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int run = threadIdx.x + RAD_THREADS * s;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[s][j] = (run >> 4) < nrow ? W[4 * run + j] : 0.f;
+    }
+  }
+  __device__ __forceinline__ float absmax() const {
+    float m = 0.f;
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) m = fmaxf(m, fabsf(v[s][j]));
+    return m;
+  }
+  // planes of the layer times sw: [row][kslot(column)], and [column][kslot(row)] (TRANS)
+  template <bool TRANS>
+  __device__ __forceinline__ void store(LayerH16& L, float sw) const {
+    typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int run = threadIdx.x + RAD_THREADS * s, o = run >> 4, u = 4 * (run & 15);
+      h4 h, l;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float x = v[s][j] * sw;   // exact: a power of two
+        h[j] = (_Float16)x;
+        l[j] = (_Float16)(x - (float)h[j]);
+      }
+      if constexpr (TRANS) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          L.p[0][u + j][kslot(o)] = h[j];
+          L.p[1][u + j][kslot(o)] = l[j];
+        }
+      } else {   // kslot keeps runs of four columns together
+        *reinterpret_cast<h4*>(&L.p[0][o][kslot(u)]) = h;
+        *reinterpret_cast<h4*>(&L.p[1][o][kslot(u)]) = l;
+      }
+    }
+  }
+};
+
+// Every weight is read once and all loads are in flight together; the layers' scales come from one reduction.
+// (A scan for the maximum and a second read per layer, W2 read for both of its orientations, took about half of
+// a small launch: the backward of 300 edges 20 us, 9.4 now.)
 template <bool BWD>
 __device__ void stage_weights(Smem<BWD>& sm, const float* __restrict__ W0, const float* __restrict__ b0,
                               const float* __restrict__ W2, const float* __restrict__ b2,
                               const float* __restrict__ W4, const float* __restrict__ b4, int nb, int nout) {
-  for (int i = threadIdx.x; i < HID * NBMAX; i += blockDim.x) {
-    const int j = i / NBMAX, k = i % NBMAX;
+  WRegs w2, w4;
+  w2.load(W2, HID);
+  if (W4) w4.load(W4, nout);
+#pragma unroll
+  for (int s = 0; s < HID * NBMAX / RAD_THREADS; ++s) {
+    const int i = threadIdx.x + RAD_THREADS * s, j = i / NBMAX, k = i % NBMAX;
     const float v = (k < nb) ? W0[j * nb + k] : 0.f;
     sm.w0[j][k] = v;
-    if (BWD) sm.w0t[k][j] = v;
+    if (BWD) sm.w0t[w0t_row(k)][j] = v;
   }
-  for (int i = threadIdx.x; i < HID; i += blockDim.x) {
+  if (threadIdx.x < HID) {
+    const int i = threadIdx.x;
     sm.b0[i] = b0[i];
     sm.b2[i] = b2[i];
     sm.b4[i] = (W4 && i < nout && b4) ? b4[i] : 0.f;
   }
-  const float w2i = stage_h16(sm.w2, sm.red, [&](int o, int u) { return W2[o * HID + u]; });
-  float w2ti = 1.f, w4i = 1.f;
-  if constexpr (BWD) w2ti = stage_h16(sm.w2t, sm.red, [&](int o, int u) { return W2[u * HID + o]; });
-  if (W4) {
-    if constexpr (BWD)   // W4^T [64 hidden][nout], zero columns beyond nout
-      w4i = stage_h16(sm.w4, sm.red, [&](int o, int u) { return u < nout ? W4[u * HID + o] : 0.f; });
-    else
-      w4i = stage_h16(sm.w4, sm.red, [&](int o, int u) { return o < nout ? W4[o * HID + u] : 0.f; });
+  float m2 = w2.absmax(), m4 = W4 ? w4.absmax() : 0.f;
+  for (int off = 32; off > 0; off >>= 1) {
+    m2 = fmaxf(m2, __shfl_xor(m2, off, 64));
+    m4 = fmaxf(m4, __shfl_xor(m4, off, 64));
   }
+  if ((threadIdx.x & 63) == 0) {
+    sm.red[threadIdx.x >> 6] = m2;
+    sm.red[RAD_WAVES + (threadIdx.x >> 6)] = m4;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < RAD_WAVES; ++w) {
+    m2 = fmaxf(m2, sm.red[w]);
+    m4 = fmaxf(m4, sm.red[RAD_WAVES + w]);
+  }
+  const float s2 = pow2_scale(m2), s4 = pow2_scale(m4);
+  w2.store<false>(sm.w2, s2);
+  if constexpr (BWD) w2.store<true>(sm.w2t, s2);
+  if (W4) w4.store<BWD>(sm.w4, s4);   // backward: W4^T [64 hidden][nout]
   if (threadIdx.x == 0) {
-    sm.winv[0] = w2i;
-    sm.winv[1] = w2ti;
-    sm.winv[2] = w4i;
+    sm.winv[0] = 1.f / s2;
+    sm.winv[1] = 1.f / s2;
+    sm.winv[2] = 1.f / s4;
   }
 }
 
@@ -196,9 +269,10 @@ __device__ __forceinline__ f4 lds4(const float* p) { return *reinterpret_cast<co
 // out = W x + b for a 64-wide layer on split-fp16 MFMA: x in the MFMA layout (x[jt][i] = unit 16 jt + 4 q + i
 // of the lane's edge r); the edge's activations scaled by a power of two from their max |x| over the four
 // lanes of the edge and split once; A operand row r of output tile ot reads K slots 8q .. 8q + 7 of
-// W row 16 ot + r from both planes; both scales undone on the fp32 result.
+// W row 16 ot + r from both planes; both scales undone on the fp32 result.  A fused last Linear of few outputs
+// works on its nout_tiles output tiles (backward: its nsteps K steps) only; the others are not written.
 __device__ __forceinline__ void dense64(const LayerH16& W, float winv, const float* b, const f4 (&x)[4], int r,
-                                        int q, f4 (&out)[4]) {
+                                        int q, f4 (&out)[4], int nout_tiles = 4, int nsteps = 2) {
   float mx = 0.f;
 #pragma unroll
   for (int jt = 0; jt < 4; ++jt)
@@ -210,22 +284,25 @@ __device__ __forceinline__ void dense64(const LayerH16& W, float winv, const flo
   h8 xh[2], xl[2];
 #pragma unroll
   for (int st = 0; st < 2; ++st) {
+    if (st >= nsteps) break;
     const float v[8] = {x[2 * st][0] * sx, x[2 * st][1] * sx, x[2 * st][2] * sx, x[2 * st][3] * sx,
                         x[2 * st + 1][0] * sx, x[2 * st + 1][1] * sx, x[2 * st + 1][2] * sx, x[2 * st + 1][3] * sx};
     split2h_pk(v, xh[st], xl[st]);
   }
-  const float f = winv / sx;   // exact: powers of two
+  const float f = winv * pow2_inverse(sx);   // exact: powers of two
 #pragma unroll
   for (int ot = 0; ot < 4; ++ot) {
+    if (ot >= nout_tiles) break;
     f4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int st = 0; st < 2; ++st) {
+      if (st >= nsteps) break;
       const h8 wh = *reinterpret_cast<const h8*>(&W.p[0][16 * ot + r][32 * st + 8 * q]);
       const h8 wl = *reinterpret_cast<const h8*>(&W.p[1][16 * ot + r][32 * st + 8 * q]);
       acc = mfma_x3(wh, wl, xh[st], xl[st], acc);
     }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) acc[i] = acc[i] * f + (b ? b[16 * ot + 4 * q + i] : 0.f);
+    acc = acc * f;
+    if (b) acc += lds4(b + 16 * ot + 4 * q);
     out[ot] = acc;
     __builtin_amdgcn_sched_barrier(0);
   }
@@ -241,9 +318,7 @@ __device__ __forceinline__ void first_layer(const Smem<BWD>& sm, const float (&e
 #pragma unroll
     for (int ks = 0; ks < NBMAX / 4; ++ks)
       if (ks < nks) acc = mfma16x16x4(sm.w0[16 * jt + r][4 * ks + q], emb[ks], acc);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) acc[i] += sm.b0[16 * jt + 4 * q + i];
-    u0[jt] = acc;
+    u0[jt] = acc + lds4(&sm.b0[16 * jt + 4 * q]);
     __builtin_amdgcn_sched_barrier(0);
   }
 }
@@ -261,33 +336,22 @@ __device__ __forceinline__ void mlp_forward(const Smem<BWD>& sm, const float (&e
   dense64(sm.w2, sm.winv[0], sm.b2, a0, r, q, u2);
 }
 
-// The basis values a lane feeds to the first product: emb[4*ks + q] for ks < nks (lane group q).
-__device__ __forceinline__ void lane_basis(float rr, int nb, float rc, int basis, int q, float (&emb)[NBMAX / 4]) {
+// The basis values a lane feeds to the first product: emb_k, k = 4 ks + q for ks < nks (lane group q), and with
+// DERIV d emb_k / dr of the same k (zero for k >= nb), which share their sine and cosine.
+template <bool DERIV>
+__device__ __forceinline__ void lane_basis(float rr, int nb, float rc, int basis, int q, float (&emb)[NBMAX / 4],
+                                           float (&demb)[NBMAX / 4]) {
 #pragma unroll
   for (int ks = 0; ks < NBMAX / 4; ++ks) {
     const int k = 4 * ks + q;
     float f = 0.f, df = 0.f;
-    if (k < nb) basis_eval<false>(rr, k, nb, rc, basis, f, df);
+    if (k < nb) basis_eval<DERIV>(rr, k, nb, rc, basis, f, df);
     emb[ks] = f;
+    if constexpr (DERIV) demb[ks] = df;
   }
 }
 
-// d emb_k / dr for the lane's rows k = 4q + i of the d-emb tile (zero for k >= nb).
-__device__ __forceinline__ void lane_basis_deriv(float rr, int nb, float rc, int basis, int q, float (&demb)[4]) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int k = 4 * q + i;
-    float f = 0.f, df = 0.f;
-    if (k < nb) basis_eval<true>(rr, k, nb, rc, basis, f, df);
-    demb[i] = df;
-  }
-}
-
-// Blocks of RAD_WAVES waves share one LDS copy of the weights; two blocks per CU give 4 waves per SIMD
-// (at most 128 VGPRs), enough to overlap the dependent layers of one 16-edge tile with other tiles.
-constexpr int RAD_WAVES = 8;
-
-__global__ __launch_bounds__(64 * RAD_WAVES, 4) void radial_mlp_forward_kernel(const float* __restrict__ rad, const float* __restrict__ W0,
+__global__ __launch_bounds__(RAD_THREADS, 4) void radial_mlp_forward_kernel(const float* __restrict__ rad, const float* __restrict__ W0,
                                                                  const float* __restrict__ b0, const float* __restrict__ W2,
                                                                  const float* __restrict__ b2, const float* __restrict__ W4,
                                                                  const float* __restrict__ b4, int nout, int nb, float rc,
@@ -307,7 +371,7 @@ __global__ __launch_bounds__(64 * RAD_WAVES, 4) void radial_mlp_forward_kernel(c
     const float rr = rr_next;
     rr_next = radius(t + tstride);
     float emb[NBMAX / 4];
-    lane_basis(rr, nb, rc, basis, q, emb);
+    lane_basis<false>(rr, nb, rc, basis, q, emb, emb);
     f4 u0[4], u2[4], a2[4];
     mlp_forward(sm, emb, nks, r, q, u0, u2);
 #pragma unroll
@@ -316,15 +380,17 @@ __global__ __launch_bounds__(64 * RAD_WAVES, 4) void radial_mlp_forward_kernel(c
       for (int i = 0; i < 4; ++i) a2[ot][i] = u2[ot][i] * sigm(u2[ot][i]);
     if (W4) {
       f4 o[4];
-      dense64(sm.w4, sm.winv[2], sm.b4, a2, r, q, o);
+      dense64(sm.w4, sm.winv[2], sm.b4, a2, r, q, o, (nout + 15) / 16);
       if (e < n_edges) {
 #pragma unroll
-        for (int ot = 0; ot < 4; ++ot)
+        for (int ot = 0; ot < 4; ++ot) {
+          if (16 * ot >= nout) break;
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             const int j = 16 * ot + 4 * q + i;
             if (j < nout) h[e * nout + j] = o[ot][i];
           }
+        }
       }
     } else if (e < n_edges) {
 #pragma unroll
@@ -335,7 +401,7 @@ __global__ __launch_bounds__(64 * RAD_WAVES, 4) void radial_mlp_forward_kernel(c
 
 // dr[e] = sum_k d emb_k/dr * (W0^T (silu'(u0) * W2^T (silu'(u2) * dh)))_k, with dh = W4^T dout when the
 // last Linear is fused.
-__global__ __launch_bounds__(64 * RAD_WAVES, 4) void radial_mlp_backward_kernel(const float* __restrict__ rad, const float* __restrict__ W0,
+__global__ __launch_bounds__(RAD_THREADS, 4) void radial_mlp_backward_kernel(const float* __restrict__ rad, const float* __restrict__ W0,
                                                                   const float* __restrict__ b0, const float* __restrict__ W2,
                                                                   const float* __restrict__ b2, const float* __restrict__ W4,
                                                                   int nout, int nb, float rc, int basis, int64_t n_edges,
@@ -351,8 +417,8 @@ __global__ __launch_bounds__(64 * RAD_WAVES, 4) void radial_mlp_backward_kernel(
     const int64_t e = 16 * t + r;
     const bool ok = e < n_edges;
     const float rr = ok ? rad[e] : 1.f;
-    float emb[NBMAX / 4];
-    lane_basis(rr, nb, rc, basis, q, emb);
+    float emb[NBMAX / 4], demb[NBMAX / 4];
+    lane_basis<true>(rr, nb, rc, basis, q, emb, demb);
     f4 u2[4];
     {
       f4 u0[4];   // recomputed below rather than held across the two 64-wide products (register pressure)
@@ -368,7 +434,7 @@ __global__ __launch_bounds__(64 * RAD_WAVES, 4) void radial_mlp_backward_kernel(
           const int j = 16 * ot + 4 * q + i;
           d[ot][i] = (ok && j < nout) ? dout[e * nout + j] : 0.f;
         }
-      dense64(sm.w4, sm.winv[2], nullptr, d, r, q, dh);
+      dense64(sm.w4, sm.winv[2], nullptr, d, r, q, dh, 4, nout > 32 ? 2 : 1);
     } else {
 #pragma unroll
       for (int ot = 0; ot < 4; ++ot) dh[ot] = ok ? ld4(dout + e * HID + 16 * ot + 4 * q) : f4{0.f, 0.f, 0.f, 0.f};
@@ -391,7 +457,7 @@ __global__ __launch_bounds__(64 * RAD_WAVES, 4) void radial_mlp_backward_kernel(
         const float s = sigm(u0[jt][i]);
         g0[jt][i] = da0[jt][i] * s * (1.f + u0[jt][i] * (1.f - s));
       }
-    // d emb[k] for k = 4q + i (rows k of one 16-row tile; k >= nb rows are zero)
+    // d emb: register i is basis function 4i + q, the lane's own demb (w0t_row; rows k >= nb are zero)
     f4 de = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int jt = 0; jt < 4; ++jt) {
@@ -399,8 +465,6 @@ __global__ __launch_bounds__(64 * RAD_WAVES, 4) void radial_mlp_backward_kernel(
 #pragma unroll
       for (int i = 0; i < 4; ++i) de = mfma16x16x4(a[i], g0[jt][i], de);
     }
-    float demb[4];   // formed here, not held across the products
-    lane_basis_deriv(rr, nb, rc, basis, q, demb);
     float part = 0.f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) part += de[i] * demb[i];
@@ -702,7 +766,7 @@ int fsc_radial_mlp_forward(int64_t n_edges, const float* r, const float* w0, con
   if (n_edges == 0) return 0;
   FSC_CHECK_ARG(r && w0 && b0 && w2 && b2 && out, "fsc_radial_mlp_forward: null pointer");
   LaunchTimer tm("radial_mlp", stream);
-  radial_mlp_forward_kernel<<<radial_grid(n_edges), 64 * RAD_WAVES, 0, stream>>>(r, w0, b0, w2, b2, w4, b4, w4 ? n_out : HID,
+  radial_mlp_forward_kernel<<<radial_grid(n_edges), RAD_THREADS, 0, stream>>>(r, w0, b0, w2, b2, w4, b4, w4 ? n_out : HID,
                                                                      n_basis, r_cut, basis, n_edges, out);
   return check_launch("radial mlp forward") ? 2 : 0;
 }
@@ -718,7 +782,7 @@ int fsc_radial_mlp_backward(int64_t n_edges, const float* r, const float* w0, co
   if (n_edges == 0) return 0;
   FSC_CHECK_ARG(r && w0 && b0 && w2 && b2 && grad_out && grad_r, "fsc_radial_mlp_backward: null pointer");
   LaunchTimer tm("radial_mlp_grad", stream);
-  radial_mlp_backward_kernel<<<radial_grid(n_edges), 64 * RAD_WAVES, 0, stream>>>(r, w0, b0, w2, b2, w4, w4 ? n_out : HID,
+  radial_mlp_backward_kernel<<<radial_grid(n_edges), RAD_THREADS, 0, stream>>>(r, w0, b0, w2, b2, w4, w4 ? n_out : HID,
                                                                       n_basis, r_cut, basis, n_edges, grad_out, grad_r);
   return check_launch("radial mlp backward") ? 2 : 0;
 }

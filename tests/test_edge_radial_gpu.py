@@ -93,6 +93,27 @@ def _periodic_graph(N, E, seed):
     return pos, src, dst, shifts * L
 
 
+# last Linear at the edges of its 16-wide output tiles and 32-wide K steps
+@pytest.mark.parametrize("P", [15, 16, 32, 33, 48, 49])
+def test_radial_mlp_with_last_linear_at_tile_edges(P):
+    test_radial_mlp_with_last_linear(P)
+
+
+def test_radial_mlp_saturated_activations():
+    """Pre-activations beyond +-88, where the sigmoid's exponential overflows: values and slopes stay finite."""
+    from fsctep_amd import ops
+    r = torch.linspace(0.3, 4.9, 333, device=DEV).requires_grad_(True)
+    w0 = torch.full((64, 8), 60.0, device=DEV) * torch.linspace(-1, 1, 64, device=DEV).unsqueeze(1)
+    w2 = torch.eye(64, device=DEV) * torch.linspace(-2, 2, 64, device=DEV)
+    z = torch.zeros(64, device=DEV)
+    h = torch.ops.fsctep.radial_mlp(r, w0, z, w2, z, None, None, 5.0, ops.BASIS["gaussian"])
+    (gr,) = torch.autograd.grad(h.sum(), r)
+    rr = r.detach().double().cpu().requires_grad_(True)
+    ref = _hidden_ref(rr, w0.double().cpu(), z.double().cpu(), w2.double().cpu(), z.double().cpu(), 5.0, 8, "gaussian")
+    (grr,) = torch.autograd.grad(ref.sum(), rr)
+    assert rel(h, ref) < 1e-5 and rel(gr, grr) < 1e-5
+
+
 @pytest.mark.parametrize("which", ["both", "n_only", "r_only"])
 def test_edge_geometry_forward_and_forces(which):
     from fsctep_amd import ops
