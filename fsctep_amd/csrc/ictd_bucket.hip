@@ -651,32 +651,33 @@ __global__ __launch_bounds__(256) void mix_tw_kernel(Dims d, const T* __restrict
 }
 
 // ---------------------------------------------------------------- channel mix, fp32
-// The fp32 forms bound by the fp32 matrix rate (157 TFLOP/s): a block of four waves takes 128 rows x 128
-// columns, wave w the rows 32w .. 32w+31.  The column operand (weights, [column][contraction]) is common to the
-// four waves and goes through LDS 32 contraction steps at a time, rows padded to 36 floats (conflict-free
-// 16-byte reads); the next slice and the wave's own rows are requested a slice (4096 MFMA cycles) ahead.
-// 60,011 elements, K 7, 128 x 128 channels (13.8 GFLOP, y and out 0.43 GB): forward
-// 279 -> 262 us, gate gradient 485 -> 270, input gradient 309 -> 170 (81 TFLOP/s), weight gradient 333 + 515 for
-// its sum -> 252 + 9; every wave read the weights from L2 itself before.
+// The fp32 forms are bound by the fp32 matrix rate (157 TFLOP/s).  These take any size; the resident kernels further
+// down are the faster ones for the sizes they hold.  A block of four waves takes 128 rows x 128 columns, wave w the
+// rows 32w .. 32w+31.  The column operand (weights, [column][contraction]) is common to the four waves and goes
+// through LDS 32 contraction steps at a time, rows padded to 36 floats (conflict-free 16-byte reads); the next slice
+// and the wave's own rows are requested a slice (4096 MFMA cycles) ahead.  60,011 elements, K 7, 128 x 128 channels
+// (13.8 GFLOP, y and out 0.43 GB): forward 279 -> 260 us, gate gradient 485 -> 272, input gradient 309 -> 171
+// (81 TFLOP/s) against every wave reading the weights from L2 itself.
 constexpr int KS = 32;          // contraction steps per slice
 constexpr int WPAD = KS + 4;
 constexpr int OPAD = 132;       // row stride of an output slice [32 columns][128 rows]; 32 * OPAD <= 128 * WPAD
 
-// The block's share of a weight slice in flight: 128 columns x 32 steps, four 16-byte pieces a thread.
+// The block's share of a weight slice in flight: 128 columns x 32 steps, four 16-byte pieces a thread.  Pieces past
+// the matrix are cleared when they are stored: a select beside the load would wait for it.
 struct WSlice {
   f4 v[4];
+  __device__ __forceinline__ static bool inside(int s, int ncol, int nk, int c0, int k0) {
+    return c0 + (int)(threadIdx.x >> 3) + 32 * s < ncol && k0 + 4 * (int)(threadIdx.x & 7) < nk;
+  }
   __device__ __forceinline__ void load(const float* __restrict__ w, int ncol, int nk, int c0, int k0) {
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
       const int c = c0 + (threadIdx.x >> 3) + 32 * s, k = k0 + 4 * (threadIdx.x & 7);
-      const bool ok = c < ncol && k < nk;
-      v[s] = ld4(w + (ok ? (int64_t)c * nk + k : 0));
-      if (!ok) v[s] = f4{0.f, 0.f, 0.f, 0.f};
+      v[s] = ld4(w + (inside(s, ncol, nk, c0, k0) ? (int64_t)c * nk + k : 0));
     }
   }
-  __device__ __forceinline__ void store(float* ws) const {
-#pragma unroll
-    for (int s = 0; s < 4; ++s) st4(ws + ((threadIdx.x >> 3) + 32 * s) * WPAD + 4 * (threadIdx.x & 7), v[s]);
+  __device__ __forceinline__ f4 piece(int s, int ncol, int nk, int c0, int k0) const {
+    return inside(s, ncol, nk, c0, k0) ? v[s] : f4{0.f, 0.f, 0.f, 0.f};
   }
 };
 
@@ -752,7 +753,9 @@ __global__ __launch_bounds__(256, 3) void mix32_kernel(Dims d, const float* __re
     while (p < pe) {
       f4 a[2][2];
       __syncthreads();   // the previous slice is read
-      w.store(ws);
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        st4(ws + ((threadIdx.x >> 3) + 32 * u) * WPAD + 4 * (threadIdx.x & 7), w.piece(u, O, I, o0, s * KS));
 #pragma unroll
       for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -881,7 +884,7 @@ __global__ __launch_bounds__(256, 3) void mix32_ty_kernel(Dims d, const float* _
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
       const int c = (threadIdx.x >> 3) + 32 * s;
-      st4(ws + (16 * (c & 7) + (c >> 3)) * WPAD + 4 * (threadIdx.x & 7), w.v[s]);
+      st4(ws + (16 * (c & 7) + (c >> 3)) * WPAD + 4 * (threadIdx.x & 7), w.piece(s, I, O, i0, k0));
     }
 #pragma unroll
     for (int h = 0; h < 2; ++h)
@@ -915,86 +918,322 @@ __global__ __launch_bounds__(256, 3) void mix32_ty_kernel(Dims d, const float* _
 }
 
 // Partial sums of grad_W[p][o][i] = sum_{(b,k)} g[b][p] go[b][o][k] y[b][p][k][i] over a range of rows.  Block
-// (split, path, 128 x 128 tile); both operands go through LDS 32 rows at a time (each read from memory once a
-// block instead of once a wave), the next rows in flight meanwhile; wave w takes a 64 x 64 quarter.
-constexpr int TPAD = 128 + 16;   // row stride of the staged rows: the four rows of an MFMA step on distinct banks
+// (split, path, 16 T x 16 T tile; T 2, 4 or 8 by the channels); both operands go through LDS 256 / T rows at a time
+// (each read from memory once a block instead of once a wave), the next rows in flight meanwhile: a thread's four
+// pieces of y and sixteen values of go are only gated or cleared when they are stored.  Wave w takes a quarter of
+// the tile.  60,011 elements, K 7, 128 x 128: 333 us with each wave loading its own operands, 252 with gates and
+// bounds applied beside the loads, 190 now; 20,011 elements at 64 x 64 on 128 x 128 tiles 98, now 28.
+template <int T>
 __global__ __launch_bounds__(256, 3) void mix32_tw_kernel(Dims d, const float* __restrict__ go,
                                                           const float* __restrict__ y, const float* __restrict__ g,
                                                           int64_t rows_per_split, float* __restrict__ part) {
-  __shared__ float gs[KS * TPAD];
-  __shared__ float ys[KS * TPAD];
+  constexpr int W = 16 * T, RS = 256 / T, WT = T / 2;
+  constexpr int TPAD = W + 16;   // row stride of the staged rows: the four rows of an MFMA step on distinct banks
+  __shared__ __align__(16) float gs[RS * TPAD];
+  __shared__ __align__(16) float ys[RS * TPAD];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, q = lane >> 4;
   const int K = d.K, P = d.P, I = d.I, O = d.O;
   const uint32_t R = (uint32_t)(d.B * K);
   const int s = blockIdx.x, p = blockIdx.y;
-  const int nib = (I + 127) / 128;
-  const int o0 = ((int)blockIdx.z / nib) * 128, i0 = ((int)blockIdx.z % nib) * 128;
+  const int nib = (I + W - 1) / W;
+  const int o0 = ((int)blockIdx.z / nib) * W, i0 = ((int)blockIdx.z % nib) * W;
   const uint32_t r0 = (uint32_t)(s * rows_per_split), r1 = (uint32_t)std::min<int64_t>(R, r0 + rows_per_split);
-  const int wo = 64 * (wave >> 1), wi = 64 * (wave & 1);
-  f4 accm[4][4];
+  const int wo = 16 * WT * (wave >> 1), wi = 16 * WT * (wave & 1);
+  f4 accm[WT][WT];
 #pragma unroll
-  for (int t = 0; t < 4; ++t)
+  for (int t = 0; t < WT; ++t)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) accm[t][j] = f4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < WT; ++j) accm[t][j] = f4{0.f, 0.f, 0.f, 0.f};
   f4 yn[4];
-  float gn[16];
-  const int ycol = i0 + 4 * (threadIdx.x & 31);
-  const int ocol = o0 + (threadIdx.x & 127), orow = __builtin_amdgcn_readfirstlane(threadIdx.x >> 7) * 16;
+  float gn[16], gate[16];
+  const int ycol = 4 * (threadIdx.x % (4 * T)), yrow = threadIdx.x / (4 * T);   // rows yrow + (64 / T) u
+  const int ocol = threadIdx.x % W;                                             // rows orow .. orow + 15
+  const int orow = 16 * (T >= 4 ? __builtin_amdgcn_readfirstlane(threadIdx.x / W) : threadIdx.x / W);
+  const bool yok = i0 + ycol < I, ook = o0 + ocol < O;
   auto request = [&](uint32_t rr) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {   // y: row (tid / 32) + 8u, 4 channels
-      const uint32_t row = rr + (threadIdx.x >> 5) + 8 * u;
-      const bool ok = row < r1 && ycol < I;
-      const uint32_t rw = ok ? row : r0, b = rw / (uint32_t)K;
-      yn[u] = ld4(y + (((int64_t)b * P + p) * K + (rw - b * K)) * I + (ok ? ycol : 0));
-      if (!ok) yn[u] = f4{0.f, 0.f, 0.f, 0.f};
+    for (int u = 0; u < 4; ++u) {
+      const uint32_t row = std::min(rr + yrow + (64 / T) * u, r1 - 1), b = row / (uint32_t)K;
+      yn[u] = ld4(y + (((int64_t)b * P + p) * K + (row - b * K)) * I + (yok ? i0 + ycol : 0));
     }
-    // go: 16 rows (the same for the wave) of one column; the element and row in it advance without divisions
-    uint32_t b = std::min(rr + orow, r1 - 1) / (uint32_t)K, k = std::min(rr + orow, r1 - 1) - b * K;
-    const float* gc = go + (int64_t)(ocol < O ? ocol : 0) * K;
+    // go: 16 rows of one column; the element and row in it advance without divisions
+    const uint32_t first = std::min(rr + orow, r1 - 1);
+    uint32_t b = first / (uint32_t)K, k = first - b * K;
+    const float* gc = go + (int64_t)(ook ? o0 + ocol : 0) * K;
 #pragma unroll
     for (int u = 0; u < 16; ++u) {
-      const float v = gc[(int64_t)b * O * K + k] * g[(int64_t)b * P + p];
-      gn[u] = rr + orow + u < r1 && ocol < O ? v : 0.f;
+      gn[u] = gc[(int64_t)b * O * K + k];
+      gate[u] = g[(int64_t)b * P + p];
       if (rr + orow + u + 1 < r1 && ++k == (uint32_t)K) { k = 0; ++b; }
     }
   };
   request(r0);
-  for (uint32_t rr = r0; rr < r1; rr += KS) {
+  for (uint32_t rr = r0; rr < r1; rr += RS) {
     __syncthreads();
 #pragma unroll
-    for (int u = 0; u < 4; ++u) st4(ys + ((threadIdx.x >> 5) + 8 * u) * TPAD + 4 * (threadIdx.x & 31), yn[u]);
+    for (int u = 0; u < 4; ++u) {
+      const int row = yrow + (64 / T) * u;
+      st4(ys + row * TPAD + ycol, yok && rr + row < r1 ? yn[u] : f4{0.f, 0.f, 0.f, 0.f});
+    }
 #pragma unroll
-    for (int u = 0; u < 16; ++u) gs[(orow + u) * TPAD + (threadIdx.x & 127)] = gn[u];
-    if (rr + KS < r1) request(rr + KS);
+    for (int u = 0; u < 16; ++u) gs[(orow + u) * TPAD + ocol] = ook && rr + orow + u < r1 ? gn[u] * gate[u] : 0.f;
+    if (rr + RS < r1) request(rr + RS);
     __syncthreads();
+    const int nrow = std::min<int>(RS, r1 - rr);   // the rows past it hold zeros
+#pragma unroll 8
+    for (int k4 = 0; k4 < nrow; k4 += 4) {
+      float a[WT], b[WT];
 #pragma unroll
-    for (int k4 = 0; k4 < KS; k4 += 4) {
-      float a[4], b[4];
+      for (int t = 0; t < WT; ++t) a[t] = gs[(k4 + q) * TPAD + wo + 16 * t + r];
 #pragma unroll
-      for (int t = 0; t < 4; ++t) a[t] = gs[(k4 + q) * TPAD + wo + 16 * t + r];
+      for (int j = 0; j < WT; ++j) b[j] = ys[(k4 + q) * TPAD + wi + 16 * j + r];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) b[j] = ys[(k4 + q) * TPAD + wi + 16 * j + r];
+      for (int t = 0; t < WT; ++t)
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) accm[t][j] = mfma16x16x4(a[t], b[j], accm[t][j]);
+        for (int j = 0; j < WT; ++j) accm[t][j] = mfma16x16x4(a[t], b[j], accm[t][j]);
     }
   }
   float* ps = part + ((int64_t)s * P + p) * O * I;
 #pragma unroll
-  for (int t = 0; t < 4; ++t)
+  for (int t = 0; t < WT; ++t)
 #pragma unroll
     for (int jj = 0; jj < 4; ++jj) {
       const int o = o0 + wo + 16 * t + 4 * q + jj;
       if (o >= O) continue;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int j = 0; j < WT; ++j) {
         const int i = i0 + wi + 16 * j + r;
         if (i < I) ps[(int64_t)o * I + i] = accm[t][j][jj];
       }
     }
+}
+
+// ---------------------------------------------------------------- channel mix, fp32, whole weight matrix resident
+// For at most 16 T input and output channels (T 2, 4, 8) one path's weight matrix fits in LDS (68 KB at 128
+// channels, two blocks a CU): it is staged once a block, and the four waves then walk row tiles of their own with
+// no barrier, the next tile's rows in flight during the products (512 MFMAs, 6.8 us at T 8).  The kernels above,
+// which bring the weights slice by slice for every 128 rows, spend half their time on starts, barriers and ends.
+// A tile is EB = 32 / K whole batch elements (row e K + k), so that a tile's outputs are contiguous.
+// 60,011 elements, K 7, 128 x 128, against the sliced kernels: forward 260 -> 214 us, gate gradient 272 -> 210;
+// 20,011 at 64 x 64: 54 -> 34, 51 -> 36 and input gradient 41 + 5 -> 38.
+struct TileRow {   // element of the tile and row in it; the rows past EB K repeat the first
+  int el, k;
+  bool ok;
+};
+// v / K for 0 <= v <= 512 and K <= 32 with mg = 65536 / K + 1 (the excess v / 65536 stays below 1 / K)
+__device__ __forceinline__ int div_k(int v, uint32_t mg) { return (int)(((uint32_t)v * mg) >> 16); }
+__device__ __forceinline__ TileRow tile_row(int rho, int K, uint32_t mg, int EB) {
+  const int el = div_k(rho, mg);
+  const bool ok = el < EB;
+  return {ok ? el : 0, ok ? rho - el * K : 0, ok};
+}
+
+// The matrix W [O][I] in LDS, zero beyond its size: ws[o][i], or transposed (TRANS) with column i of the product in
+// row 16 (i % T) + i / T, so that a lane's T tiles are T consecutive columns.
+template <int T, bool TRANS>
+__device__ __forceinline__ void stage_matrix(const float* __restrict__ W, int O, int I, float* ws) {
+  constexpr int LD = 16 * T + 4;
+#pragma unroll
+  for (int s = 0; s < T * T / 4; ++s) {
+    const int idx = threadIdx.x + 256 * s, o = idx / (4 * T), i = 4 * (idx % (4 * T));
+    f4 v = {0.f, 0.f, 0.f, 0.f};
+    if (o < O && i < I) v = ld4(W + (int64_t)o * I + i);
+    if constexpr (TRANS) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) ws[(16 * ((i + u) % T) + (i + u) / T) * LD + o] = v[u];
+    } else {
+      st4(ws + o * LD + i, v);
+    }
+  }
+}
+
+// MODE 0: out[b][o][k] (+)= g[b] sum_i y[b][k][i] W[o][i]  (one path; src = y)
+// MODE 1: grad_g[b][p] (+)= sum_{k,i} y[b][p][k][i] u[b][k][i], u = sum_o go[b][o][k] W[p][o][i]  (path blockIdx.y,
+//         src = go; contracting over o first meets y, whose rows are contiguous, after the products)
+// MODE 2: grad_y[b][p][k][i] (+)= g[b][p] u[b][k][i]  (path blockIdx.y, src = go)
+template <int T, int MODE>
+__global__ __launch_bounds__(256, 2) void mix32_resident_kernel(Dims d, int EB, const float* __restrict__ src,
+                                                                const float* __restrict__ W,
+                                                                const float* __restrict__ g,
+                                                                const float* __restrict__ y, float* __restrict__ dst,
+                                                                int acc) {
+  constexpr int LD = 16 * T + 4, BLD = 36;
+  __shared__ __align__(16) float ws[16 * T * LD];
+  __shared__ __align__(16) float tr[MODE == 2 ? 1 : 4][MODE == 0 ? 16 * BLD : 32];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, q = lane >> 4;
+  const int K = d.K, P = d.P, I = d.I, O = d.O, p = MODE == 0 ? 0 : (int)blockIdx.y;
+  stage_matrix<T, MODE != 0>(W + (int64_t)p * O * I, O, I, ws);
+  __syncthreads();
+  const int nk = MODE != 0 ? O : I;                                   // contraction length
+  const int64_t sstride = MODE != 0 ? (int64_t)O * K : (int64_t)K * I;   // an element of src
+  const uint32_t mg = 65536u / (uint32_t)K + 1;
+  const TileRow ar[2] = {tile_row(r, K, mg, EB), tile_row(16 + r, K, mg, EB)};
+  const int64_t ntiles = (d.B + EB - 1) / EB, tstep = (int64_t)gridDim.x * 4;
+  // one register set: a step's rows are requested for the next tile as soon as its products are issued
+  f4 a[2][T];
+  float gt[2] = {1.f, 1.f};
+  const float* sp[2];
+  auto rows_of = [&](int64_t tile) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int64_t b = std::min<int64_t>(tile * EB + ar[t].el, d.B - 1);
+      if constexpr (MODE == 0) gt[t] = g[b];
+      sp[t] = src + b * sstride + (MODE != 0 ? ar[t].k : ar[t].k * I);
+    }
+  };
+  auto request = [&](int h) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int k = 16 * h + 4 * q, kc = k < nk ? k : 0;
+      if constexpr (MODE != 0) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) a[t][h][u] = sp[t][(int64_t)(kc + u) * K];
+      } else {
+        a[t][h] = ld4(sp[t] + kc);
+      }
+    }
+  };
+  int64_t tile = (int64_t)blockIdx.x * 4 + wave;
+  if (tile >= ntiles) return;   // no barrier follows
+  rows_of(tile);
+#pragma unroll
+  for (int h = 0; h < T; ++h) request(h);
+  for (; tile < ntiles; tile += tstep) {
+    f4 accm[2][T];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int j = 0; j < T; ++j) accm[t][j] = f4{0.f, 0.f, 0.f, 0.f};
+    const float gate0 = gt[0], gate1 = gt[1];
+    rows_of(std::min(tile + tstep, ntiles - 1));
+#pragma unroll
+    for (int h = 0; h < T; ++h) {
+      f4 av[2] = {a[0][h], a[1][h]};
+      if constexpr (MODE == 0) {
+        av[0] = av[0] * gate0;
+        av[1] = av[1] * gate1;
+      }
+      if (16 * h + 4 * q >= nk) av[0] = av[1] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < T; ++j) {
+        const f4 bv = ld4(ws + (16 * j + r) * LD + 16 * h + 4 * q);
+#pragma unroll
+        for (int t = 0; t < 2; ++t) accm[t][j] = mfma_k16(av[t], bv, accm[t][j]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      request(h);
+    }
+    const int64_t b0 = tile * EB;
+    const int nel = (int)std::min<int64_t>(EB, d.B - b0);
+    uint32_t mge = mg;
+    asm volatile("" : "+s"(mge));   // row indices are formed anew for each tile, not held across the products
+    if constexpr (MODE == 0) {
+      // out[b][o][k] holds an element's rows side by side: 16 columns at a time turn through LDS and leave in runs
+      // of 16 K floats an element (a store per register would write 4 bytes every 4 K)
+      float* ob = dst + b0 * O * K;
+      int lo[8], oo[8], cc[8];   // place in LDS, place in the output and column of the lane's 8 values of a slice
+      {
+        const int run = 16 * K;
+        int el = div_k(lane >> 4, mge), rem = lane - el * run, c = div_k(rem, mge), k = rem - c * K;
+        const int dk = 64 - div_k(64, mge) * K, dc = div_k(64, mge);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          lo[u] = c * BLD + el * K + k;
+          oo[u] = (el * O + c) * K + k;
+          cc[u] = el < nel ? c : 1 << 20;
+          k += dk;   // 64 values on, with carries
+          c += dc;
+          if (k >= K) { k -= K; ++c; }
+          while (c >= 16) { c -= 16; ++el; }
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < T; ++j) {
+        __builtin_amdgcn_wave_barrier();   // the LDS operations of a wave are in order
+#pragma unroll
+        for (int t = 0; t < 2; ++t) st4(&tr[wave][r * BLD + 16 * t + 4 * q], accm[t][j]);
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+          if (cc[u] + 16 * j < O) put(ob + oo[u] + 16 * j * K, tr[wave][lo[u]], acc);
+      }
+    } else if constexpr (MODE == 1) {
+      float rowsum[8];
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) {
+          const TileRow w = tile_row(16 * t + 4 * q + jj, K, mge, EB);
+          const float* yp = y + (((b0 + (w.el < nel ? w.el : 0)) * P + p) * K + w.k) * I;
+          float v = 0.f;
+          if constexpr (T >= 4) {
+#pragma unroll
+            for (int hh = 0; hh < T / 4; ++hh) {
+              const bool iv = T * r + 4 * hh < I;   // I % 4 == 0
+              const f4 yv = ld4(yp + (iv ? T * r + 4 * hh : 0));
+#pragma unroll
+              for (int u = 0; u < 4; ++u) v += iv ? accm[t][4 * hh + u][jj] * yv[u] : 0.f;
+            }
+          } else {
+#pragma unroll
+            for (int j = 0; j < T; ++j) {
+              const int i = T * r + j;
+              const float yv = yp[std::min(i, I - 1)];
+              v += i < I ? accm[t][j][jj] * yv : 0.f;
+            }
+          }
+          rowsum[4 * t + jj] = v;
+        }
+      // over the 16 column lanes by halving exchanges: lane bits 3, 2, 1 choose the half of the rows kept
+#pragma unroll
+      for (int n = 4, off = 8; n > 0; n >>= 1, off >>= 1) {
+        const bool hi = lane & off;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (i < n) {
+            const float mine = hi ? rowsum[i + n] : rowsum[i], other = hi ? rowsum[i] : rowsum[i + n];
+            rowsum[i] = mine + __shfl_xor(other, off, 64);
+          }
+      }
+      rowsum[0] += __shfl_xor(rowsum[0], 1, 64);
+      const int i8 = (lane >> 1) & 7;   // 4 t + jj of the row this lane holds
+      __builtin_amdgcn_wave_barrier();
+      if (!(lane & 1)) tr[wave][16 * (i8 >> 2) + 4 * q + (i8 & 3)] = rowsum[0];
+      __builtin_amdgcn_wave_barrier();
+      if (lane < nel) {
+        float v = 0.f;
+        for (int k = 0; k < K; ++k) v += tr[wave][lane * K + k];
+        put(dst + (b0 + lane) * P + p, v, acc);
+      }
+    } else {
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) {
+          const TileRow w = tile_row(16 * t + 4 * q + jj, K, mge, EB);
+          if (!w.ok || w.el >= nel) continue;
+          const int64_t b = b0 + w.el;
+          const float gate = g[b * P + p];
+          float* o = dst + ((b * P + p) * K + w.k) * I + T * r;
+          if constexpr (T >= 4) {
+#pragma unroll
+            for (int hh = 0; hh < T / 4; ++hh)
+              if (T * r + 4 * hh < I) {   // I % 4 == 0
+                f4 v = {accm[t][4 * hh][jj], accm[t][4 * hh + 1][jj], accm[t][4 * hh + 2][jj], accm[t][4 * hh + 3][jj]};
+                v = v * gate;
+                if (acc) v = ld4(o + 4 * hh) + v;
+                st4(o + 4 * hh, v);
+              }
+          } else {
+#pragma unroll
+            for (int j = 0; j < T; ++j)
+              if (T * r + j < I) put(o + j, accm[t][j][jj] * gate, acc);
+          }
+        }
+    }
+  }
 }
 
 // ---------------------------------------------------------------- host side
@@ -1017,6 +1256,33 @@ size_t proj_t_lds(const Dims& d, bool do_u, size_t elem) {
   const int PK = d.P * d.K, MN = d.m1 * d.m2;
   const size_t main = (size_t)(MN * PK + 4 * (IC * d.m1 + IC * (PK + 1) + d.m1 * PK)) * elem;
   return do_u ? std::max(main, (size_t)4 * MN * PK * elem) : main;
+}
+
+// Tile width of the resident form, 0 where it does not apply: channels within one matrix of 128 x 128, whole
+// elements filling at least 24 of a tile's 32 rows (every K up to 10; 17 rows of 32 at K 17 would double the work).
+int resident_width(const Dims& d) {
+  const int eb = 32 / d.K, c = std::max(d.I, d.O);
+  if (d.K > 32 || eb * d.K < 24 || c > 128) return 0;
+  return c <= 32 ? 2 : c <= 64 ? 4 : 8;
+}
+
+template <int MODE>
+void launch_resident(const Dims& d, int t, const float* src, const float* w, const float* g, const float* y, float* dst,
+                     int acc, hipStream_t st) {
+  const int eb = 32 / d.K;
+  const int64_t blocks = ((d.B + eb - 1) / eb + 3) / 4, paths = MODE == 0 ? 1 : d.P;
+  // as many blocks as are resident at once: the matrix is staged once in each
+  const int64_t cap = std::max<int64_t>(1, (t == 8 ? 512 : t == 4 ? 1024 : 2048) / paths);
+  const dim3 grid((unsigned)std::min(blocks, cap), (unsigned)paths);
+  if constexpr (MODE != 2)
+    if (t == 8) {
+      mix32_resident_kernel<8, MODE><<<grid, 256, 0, st>>>(d, eb, src, w, g, y, dst, acc);
+      return;
+    }
+  if (t == 4)
+    mix32_resident_kernel<4, MODE><<<grid, 256, 0, st>>>(d, eb, src, w, g, y, dst, acc);
+  else
+    mix32_resident_kernel<2, MODE><<<grid, 256, 0, st>>>(d, eb, src, w, g, y, dst, acc);
 }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
@@ -1118,9 +1384,13 @@ int mix(int64_t B, int32_t P, int32_t K, int32_t I, int32_t O, const T* y, const
   if (check_dims(d, false)) return 1;
   if (B == 0) return 0;
   const dim3 grid((unsigned)((B * K + 127) / 128), (unsigned)((O + 127) / 128));
-  if constexpr (std::is_same_v<T, float>)
-    mix32_kernel<false><<<grid, 256, 0, st>>>(d, y, w, gates, nullptr, out, accumulate);
-  else
+  if constexpr (std::is_same_v<T, float>) {
+    const int t = P == 1 ? resident_width(d) : 0;   // several paths add up in one product: slice by slice
+    if (t)
+      launch_resident<0>(d, t, y, w, gates, nullptr, out, accumulate, st);
+    else
+      mix32_kernel<false><<<grid, 256, 0, st>>>(d, y, w, gates, nullptr, out, accumulate);
+  } else
     mix_kernel<T, false><<<grid, 256, 0, st>>>(d, y, w, gates, nullptr, out, accumulate);
   return check_launch("bucket mix") ? 2 : 0;
 }
@@ -1133,19 +1403,28 @@ int mix_transpose_g(int64_t B, int32_t P, int32_t K, int32_t I, int32_t O, const
   if (B == 0) return 0;
   const int BB = 128 / K;
   const dim3 grid((unsigned)((B + BB - 1) / BB), (unsigned)P);
-  if constexpr (std::is_same_v<T, float>)
-    mix32_kernel<true><<<grid, 256, 0, st>>>(d, y, w, nullptr, grad_out, grad_g, accumulate);
-  else
+  if constexpr (std::is_same_v<T, float>) {
+    if (const int t = resident_width(d))
+      launch_resident<1>(d, t, grad_out, w, nullptr, y, grad_g, accumulate, st);
+    else
+      mix32_kernel<true><<<grid, 256, 0, st>>>(d, y, w, nullptr, grad_out, grad_g, accumulate);
+  } else
     mix_kernel<T, true><<<grid, 256, 0, st>>>(d, y, w, nullptr, grad_out, grad_g, accumulate);
   return check_launch("bucket mix_transpose_g") ? 2 : 0;
 }
 
+// Tile of the weight gradient (16 T channels a side; the fp64 kernel's is 128 whatever T) and its row splits: about
+// 768 blocks, three a CU, of at least 64 rows (256 rows a split left 700 elements on 3 to 20 blocks: 57 us, 13 now).
+int mix_tw_tile(int32_t I, int32_t O) {
+  const int c = std::max(I, O);
+  return c <= 32 ? 2 : c <= 64 ? 4 : 8;
+}
 int64_t mix_tw_splits(int64_t B, int32_t P, int32_t K, int32_t I, int32_t O, int64_t* rows_per_split) {
   const int64_t R = std::max<int64_t>(B * K, 1);
   const int64_t tiles = (int64_t)P * ((O + 127) / 128) * ((I + 127) / 128);
-  const int64_t want = std::max<int64_t>(1, 768 / tiles);   // three blocks a CU
-  int64_t rps = std::max<int64_t>(256, (R + want - 1) / want);
-  rps = (rps + 15) / 16 * 16;
+  const int64_t want = std::max<int64_t>(1, 768 / tiles);
+  int64_t rps = std::max<int64_t>(64, (R + want - 1) / want);
+  rps = (rps + 31) / 32 * 32;
   *rows_per_split = rps;
   return (R + rps - 1) / rps;
 }
@@ -1165,6 +1444,14 @@ int mix_transpose_y(int64_t B, int32_t P, int32_t K, int32_t I, int32_t O, const
   const Dims d{B, I, 0, 0, P, K, O};
   if (check_dims(d, false)) return 1;
   if (B == 0) return 0;
+  if constexpr (std::is_same_v<T, float>) {
+    // at 128 channels the sliced kernel is the faster of the two (60,011 elements, K 7: 171 + 5 us for its transposed
+    // weights against 192), below it the resident one (20,011 at 64: 27 + 5 against 24)
+    if (const int t = resident_width(d); t && t < 8) {
+      launch_resident<2>(d, t, grad_out, w, gates, nullptr, grad_y, accumulate, st);
+      return check_launch("bucket mix_transpose_y") ? 2 : 0;
+    }
+  }
   const int64_t nw = (int64_t)P * O * I;
   transpose_w_kernel<T><<<(unsigned)std::min<int64_t>((nw + 255) / 256, 4096), 256, 0, st>>>(P, O, I, w, workspace);
   if (check_launch("bucket transpose_w")) return 2;
@@ -1190,7 +1477,11 @@ int mix_transpose_w(int64_t B, int32_t P, int32_t K, int32_t I, int32_t O, const
   const int64_t ns = mix_tw_splits(B, P, K, I, O, &rps);
   const dim3 grid((unsigned)ns, (unsigned)P, (unsigned)(((O + 127) / 128) * ((I + 127) / 128)));
   if constexpr (std::is_same_v<T, float>)
-    mix32_tw_kernel<<<grid, 256, 0, st>>>(d, grad_out, y, gates, rps, workspace);
+    switch (mix_tw_tile(I, O)) {
+      case 2: mix32_tw_kernel<2><<<grid, 256, 0, st>>>(d, grad_out, y, gates, rps, workspace); break;
+      case 4: mix32_tw_kernel<4><<<grid, 256, 0, st>>>(d, grad_out, y, gates, rps, workspace); break;
+      default: mix32_tw_kernel<8><<<grid, 256, 0, st>>>(d, grad_out, y, gates, rps, workspace);
+    }
   else
     mix_tw_kernel<T><<<grid, 256, 0, st>>>(d, grad_out, y, gates, rps, workspace);
   if (check_launch("bucket mix_transpose_w")) return 2;
