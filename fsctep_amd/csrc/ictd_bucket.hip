@@ -1010,13 +1010,18 @@ __global__ __launch_bounds__(256, 3) void mix32_tw_kernel(Dims d, const float* _
 }
 
 // ---------------------------------------------------------------- channel mix, fp32, whole weight matrix resident
-// For at most 16 T input and output channels (T 2, 4, 8) one path's weight matrix fits in LDS (68 KB at 128
+// For at most 16 T input and output channels (T 2, 4, 8) one path's weight matrix fits in LDS (70 KB at 128
 // channels, two blocks a CU): it is staged once a block, and the four waves then walk row tiles of their own with
-// no barrier, the next tile's rows in flight during the products (512 MFMAs, 6.8 us at T 8).  The kernels above,
-// which bring the weights slice by slice for every 128 rows, spend half their time on starts, barriers and ends.
+// no barrier, the next tile's rows in flight during the products.  The products are split-fp16 (common.h): the matrix
+// is scaled by one power of two and staged as two fp16 planes, each row by the power of two of its own largest value
+// (both undone on the result), 3 MFMAs of 16 cycles a 32-deep step against 8 of 32 on the fp32 MFMA, which bound the
+// fp32 form of these kernels.  Error against 64 bits, 3,011 elements, outputs / gradients of the
+// gates: 1.5e-7 / 2.5e-7 at 128 channels, 1.1e-7 / 1.9e-7 at 32 (fp32 MFMA: 2.1e-7 / 2.9e-7, 1.2e-7 / 3.2e-7); a row
+// or matrix with a non-finite entry gives non-finite results and leaves the other rows' alone.
 // A tile is EB = 32 / K whole batch elements (row e K + k), so that a tile's outputs are contiguous.
-// 60,011 elements, K 7, 128 x 128, against the sliced kernels: forward 260 -> 214 us, gate gradient 272 -> 210;
-// 20,011 at 64 x 64: 54 -> 34, 51 -> 36 and input gradient 41 + 5 -> 38.
+// 60,011 elements, K 7, 128 x 128, sliced kernels / resident with fp32 products / this: forward 260 / 214 / 118 us,
+// gate gradient 272 / 210 / 165, input gradient 171 + 5 / 190 / 168 (the last two read go in 4-byte pieces, element
+// columns 4 K apart, and wait for them); 20,011 at 64 x 64: 54 / 34 / 27, 51 / 36 / 27, 41 + 5 / 38 / 35.
 struct TileRow {   // element of the tile and row in it; the rows past EB K repeat the first
   int el, k;
   bool ok;
@@ -1029,23 +1034,55 @@ __device__ __forceinline__ TileRow tile_row(int rho, int K, uint32_t mg, int EB)
   return {ok ? el : 0, ok ? rho - el * K : 0, ok};
 }
 
-// The matrix W [O][I] in LDS, zero beyond its size: ws[o][i], or transposed (TRANS) with column i of the product in
-// row 16 (i % T) + i / T, so that a lane's T tiles are T consecutive columns.
+__device__ __forceinline__ float finite_abs(float v) { return fabsf(v) <= 3.402823466e38f ? fabsf(v) : 0.f; }
+
+// The matrix W [O][I] in LDS as the fp16 planes of W sw, zero beyond its size: ws[plane][o][i], or transposed (TRANS)
+// with column i of the product in row 16 (i % T) + i / T, so that a lane's T tiles are T consecutive columns.
+// sw is the power of two of the largest finite |W|; returns 1/sw.  Ends with a barrier.
 template <int T, bool TRANS>
-__device__ __forceinline__ void stage_matrix(const float* __restrict__ W, int O, int I, float* ws) {
-  constexpr int LD = 16 * T + 4;
+__device__ __forceinline__ float stage_matrix(const float* __restrict__ W, int O, int I,
+                                              _Float16 (&ws)[2][16 * T][16 * T + 8], float (&red)[4]) {
+  typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+  constexpr int NP = T * T / 4;
+  f4 v[NP];
+  float mx = 0.f;
 #pragma unroll
-  for (int s = 0; s < T * T / 4; ++s) {
+  for (int s = 0; s < NP; ++s) {
     const int idx = threadIdx.x + 256 * s, o = idx / (4 * T), i = 4 * (idx % (4 * T));
-    f4 v = {0.f, 0.f, 0.f, 0.f};
-    if (o < O && i < I) v = ld4(W + (int64_t)o * I + i);
+    v[s] = ld4(W + (o < O && i < I ? (int64_t)o * I + i : 0));
+  }
+#pragma unroll
+  for (int s = 0; s < NP; ++s)
+#pragma unroll
+    for (int u = 0; u < 4; ++u) mx = fmaxf(mx, finite_abs(v[s][u]));
+  for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
+  __syncthreads();
+  const float sw = pow2_scale(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
+#pragma unroll
+  for (int s = 0; s < NP; ++s) {
+    const int idx = threadIdx.x + 256 * s, o = idx / (4 * T), i = 4 * (idx % (4 * T));
+    const bool ok = o < O && i < I;
+    h4 h, l;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const float x = ok ? v[s][u] * sw : 0.f;
+      h[u] = (_Float16)x;
+      l[u] = (_Float16)(x - (float)h[u]);
+    }
     if constexpr (TRANS) {
 #pragma unroll
-      for (int u = 0; u < 4; ++u) ws[(16 * ((i + u) % T) + (i + u) / T) * LD + o] = v[u];
+      for (int u = 0; u < 4; ++u) {
+        ws[0][16 * ((i + u) % T) + (i + u) / T][o] = h[u];
+        ws[1][16 * ((i + u) % T) + (i + u) / T][o] = l[u];
+      }
     } else {
-      st4(ws + o * LD + i, v);
+      *reinterpret_cast<h4*>(&ws[0][o][i]) = h;
+      *reinterpret_cast<h4*>(&ws[1][o][i]) = l;
     }
   }
+  __syncthreads();
+  return 1.f / sw;
 }
 
 // MODE 0: out[b][o][k] (+)= g[b] sum_i y[b][k][i] W[o][i]  (one path; src = y)
@@ -1058,73 +1095,94 @@ __global__ __launch_bounds__(256, 2) void mix32_resident_kernel(Dims d, int EB, 
                                                                 const float* __restrict__ g,
                                                                 const float* __restrict__ y, float* __restrict__ dst,
                                                                 int acc) {
-  constexpr int LD = 16 * T + 4, BLD = 36;
-  __shared__ __align__(16) float ws[16 * T * LD];
+  constexpr int BLD = 36, HS = T / 2;   // HS: 32-deep contraction steps
+  __shared__ __align__(16) _Float16 ws[2][16 * T][16 * T + 8];
+  __shared__ float red[4];
   __shared__ __align__(16) float tr[MODE == 2 ? 1 : 4][MODE == 0 ? 16 * BLD : 32];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, q = lane >> 4;
   const int K = d.K, P = d.P, I = d.I, O = d.O, p = MODE == 0 ? 0 : (int)blockIdx.y;
-  stage_matrix<T, MODE != 0>(W + (int64_t)p * O * I, O, I, ws);
-  __syncthreads();
+  const float winv = stage_matrix<T, MODE != 0>(W + (int64_t)p * O * I, O, I, ws, red);
   const int nk = MODE != 0 ? O : I;                                   // contraction length
   const int64_t sstride = MODE != 0 ? (int64_t)O * K : (int64_t)K * I;   // an element of src
   const uint32_t mg = 65536u / (uint32_t)K + 1;
   const TileRow ar[2] = {tile_row(r, K, mg, EB), tile_row(16 + r, K, mg, EB)};
   const int64_t ntiles = (d.B + EB - 1) / EB, tstep = (int64_t)gridDim.x * 4;
-  // one register set: a step's rows are requested for the next tile as soon as its products are issued
-  f4 a[2][T];
+  f4 a[2][T];   // the lane's rows: contraction steps 32 h + 8 q + 4 e .. + 3 in a[.][2 h + e]
   float gt[2] = {1.f, 1.f};
-  const float* sp[2];
-  auto rows_of = [&](int64_t tile) {
+  auto request = [&](int64_t tile) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       const int64_t b = std::min<int64_t>(tile * EB + ar[t].el, d.B - 1);
       if constexpr (MODE == 0) gt[t] = g[b];
-      sp[t] = src + b * sstride + (MODE != 0 ? ar[t].k : ar[t].k * I);
-    }
-  };
-  auto request = [&](int h) {
+      const float* sp = src + b * sstride + (MODE != 0 ? ar[t].k : ar[t].k * I);
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int k = 16 * h + 4 * q, kc = k < nk ? k : 0;
-      if constexpr (MODE != 0) {
+      for (int h = 0; h < T; ++h) {
+        const int k = 32 * (h >> 1) + 8 * q + 4 * (h & 1), kc = k < nk ? k : 0;
+        if constexpr (MODE != 0) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) a[t][h][u] = sp[t][(int64_t)(kc + u) * K];
-      } else {
-        a[t][h] = ld4(sp[t] + kc);
+          for (int u = 0; u < 4; ++u) a[t][h][u] = sp[(int64_t)(kc + u) * K];
+        } else {
+          a[t][h] = ld4(sp + kc);
+        }
       }
     }
   };
   int64_t tile = (int64_t)blockIdx.x * 4 + wave;
   if (tile >= ntiles) return;   // no barrier follows
-  rows_of(tile);
-#pragma unroll
-  for (int h = 0; h < T; ++h) request(h);
+  request(tile);
   for (; tile < ntiles; tile += tstep) {
+    // the rows split, each by the power of two of its largest finite value (its values sit in four lanes); fr undoes
+    // the scales on the row's results and applies the gate
+    h8 xh[2][HS], xl[2][HS];
+    float fr[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      float mx = 0.f;
+#pragma unroll
+      for (int h = 0; h < T; ++h) {
+        if (32 * (h >> 1) + 8 * q + 4 * (h & 1) >= nk) a[t][h] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int u = 0; u < 4; ++u) mx = fmaxf(mx, finite_abs(a[t][h][u]));
+      }
+      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      const float sr = pow2_scale(mx);
+#pragma unroll
+      for (int h = 0; h < HS; ++h) {
+        const float v[8] = {a[t][2 * h][0],     a[t][2 * h][1],     a[t][2 * h][2],     a[t][2 * h][3],
+                            a[t][2 * h + 1][0], a[t][2 * h + 1][1], a[t][2 * h + 1][2], a[t][2 * h + 1][3]};
+        split2h(v, sr, xh[t][h], xl[t][h]);
+      }
+      fr[t] = winv / sr;   // exact: powers of two
+      if constexpr (MODE == 0) fr[t] *= gt[t];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    request(std::min(tile + tstep, ntiles - 1));
+    __builtin_amdgcn_sched_barrier(0);
     f4 accm[2][T];
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int j = 0; j < T; ++j) accm[t][j] = f4{0.f, 0.f, 0.f, 0.f};
-    const float gate0 = gt[0], gate1 = gt[1];
-    rows_of(std::min(tile + tstep, ntiles - 1));
 #pragma unroll
-    for (int h = 0; h < T; ++h) {
-      f4 av[2] = {a[0][h], a[1][h]};
-      if constexpr (MODE == 0) {
-        av[0] = av[0] * gate0;
-        av[1] = av[1] * gate1;
-      }
-      if (16 * h + 4 * q >= nk) av[0] = av[1] = f4{0.f, 0.f, 0.f, 0.f};
+    for (int h = 0; h < HS; ++h)
 #pragma unroll
       for (int j = 0; j < T; ++j) {
-        const f4 bv = ld4(ws + (16 * j + r) * LD + 16 * h + 4 * q);
+        const h8 wh = *reinterpret_cast<const h8*>(&ws[0][16 * j + r][32 * h + 8 * q]);
+        const h8 wl = *reinterpret_cast<const h8*>(&ws[1][16 * j + r][32 * h + 8 * q]);
 #pragma unroll
-        for (int t = 0; t < 2; ++t) accm[t][j] = mfma_k16(av[t], bv, accm[t][j]);
+        for (int t = 0; t < 2; ++t) accm[t][j] = mfma_x3(xh[t][h], xl[t][h], wh, wl, accm[t][j]);
       }
-      __builtin_amdgcn_sched_barrier(0);
-      request(h);
-    }
+    // result register jj of lane group q is row 4 q + jj of the tile: its factor is held by lane 4 q + jj
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int jj = 0; jj < 4; ++jj) {
+        const float f = __shfl(fr[t], 4 * q + jj, 64);
+#pragma unroll
+        for (int j = 0; j < T; ++j) accm[t][j][jj] *= f;
+      }
     const int64_t b0 = tile * EB;
     const int nel = (int)std::min<int64_t>(EB, d.B - b0);
     uint32_t mge = mg;
@@ -1185,6 +1243,7 @@ __global__ __launch_bounds__(256, 2) void mix32_resident_kernel(Dims d, int EB, 
             }
           }
           rowsum[4 * t + jj] = v;
+          if (jj & 1) __builtin_amdgcn_sched_barrier(0);   // two rows of y in flight, not all eight (registers)
         }
       // over the 16 column lanes by halving exchanges: lane bits 3, 2, 1 choose the half of the rows kept
 #pragma unroll
@@ -1274,12 +1333,9 @@ void launch_resident(const Dims& d, int t, const float* src, const float* w, con
   // as many blocks as are resident at once: the matrix is staged once in each
   const int64_t cap = std::max<int64_t>(1, (t == 8 ? 512 : t == 4 ? 1024 : 2048) / paths);
   const dim3 grid((unsigned)std::min(blocks, cap), (unsigned)paths);
-  if constexpr (MODE != 2)
-    if (t == 8) {
-      mix32_resident_kernel<8, MODE><<<grid, 256, 0, st>>>(d, eb, src, w, g, y, dst, acc);
-      return;
-    }
-  if (t == 4)
+  if (t == 8)
+    mix32_resident_kernel<8, MODE><<<grid, 256, 0, st>>>(d, eb, src, w, g, y, dst, acc);
+  else if (t == 4)
     mix32_resident_kernel<4, MODE><<<grid, 256, 0, st>>>(d, eb, src, w, g, y, dst, acc);
   else
     mix32_resident_kernel<2, MODE><<<grid, 256, 0, st>>>(d, eb, src, w, g, y, dst, acc);
@@ -1445,9 +1501,7 @@ int mix_transpose_y(int64_t B, int32_t P, int32_t K, int32_t I, int32_t O, const
   if (check_dims(d, false)) return 1;
   if (B == 0) return 0;
   if constexpr (std::is_same_v<T, float>) {
-    // at 128 channels the sliced kernel is the faster of the two (60,011 elements, K 7: 171 + 5 us for its transposed
-    // weights against 192), below it the resident one (20,011 at 64: 27 + 5 against 24)
-    if (const int t = resident_width(d); t && t < 8) {
+    if (const int t = resident_width(d)) {
       launch_resident<2>(d, t, grad_out, w, gates, nullptr, grad_y, accumulate, st);
       return check_launch("bucket mix_transpose_y") ? 2 : 0;
     }

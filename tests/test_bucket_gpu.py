@@ -106,6 +106,33 @@ def test_mix_ops_at_tile_edges(case):
     test_mix_ops(case, torch.float32)
 
 
+@pytest.mark.parametrize("C", [32, 64, 128])
+def test_mix_ops_rows_of_any_magnitude(C):
+    """Rows from 1e-15 to 1e15 keep their own relative accuracy (each row has its own scale), and an infinite row
+    leaves every other row's result alone."""
+    E, B, K = ext(), 75, 3
+    mag = torch.logspace(-15, 15, B, dtype=torch.float64).view(B, 1, 1)
+    y, w, g = rnd(B, 1, K, C, seed=1) * mag.unsqueeze(-1), rnd(1, C, C, seed=2), rnd(B, 1, seed=3)
+    go = rnd(B, C, K, seed=4) * mag
+    bad = 41
+    yb, gob = gpu(y), gpu(go)
+    yb[bad, 0, 1, 5] = float("inf")
+    gob[bad, 7, 2] = float("-inf")
+    unit = y / mag.unsqueeze(-1)
+    ref = {"out": BR.mix_forward(y, w, g), "y": BR.mix_transpose(go, y, w, g)[0], "g": BR.mix_transpose(go, unit, w, g)[2]}
+    got = {"out": E.mix_bucket_forward(yb, gpu(w), gpu(g)), "y": E.mix_bucket_transpose_y(gob, gpu(w), gpu(g)),
+           "g": E.mix_bucket_transpose_g(gob, gpu(unit), gpu(w))}
+    keep = torch.arange(B) != bad
+    for k, r in ref.items():
+        x = got[k].double().cpu()
+        assert not torch.isfinite(x[bad]).all()
+        scale = r[keep].abs().reshape(B - 1, -1).amax(1).clamp_min(1e-30)
+        # the gate gradient is one cancelling sum over K C terms: relative to the size of its terms, sqrt(K C) |go| |y W|
+        if k == "g":
+            scale = mag.reshape(B)[keep] * (K * C) ** 0.5 * C ** 0.5
+        assert float(((x - r)[keep].abs().reshape(B - 1, -1).amax(1) / scale).max()) < TOL
+
+
 @pytest.mark.parametrize("case", [(5, 16, 9, 9, 1, 16), (9, 20, 3, 8, 1, 17), (7, 12, 9, 9, 4, 8), (6, 4, 1, 9, 3, 11),
                                   (3, 36, 5, 1, 7, 7), (8193, 8, 3, 5, 1, 64), (11, 18, 3, 3, 2, 3)])
 def test_direction_gradient_at_tile_edges(case):
