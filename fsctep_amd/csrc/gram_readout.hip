@@ -656,6 +656,131 @@ __global__ __launch_bounds__(512, D == 1 ? 4 : 2) void backward_h16_kernel(int64
   }
 }
 
+// The backward for few nodes.  With one or two node tiles the kernel above leaves nC/16 workgroups walking the
+// column blocks one after another, each step waiting for its block of weights (32 nodes, nC 192: 12 workgroups, 12
+// steps, 39 us).  Here a workgroup takes R rows of a row block and G = 16 / R column blocks a step: the same work and
+// staging a step, 1/G of the steps, G times the workgroups.  Four waves of 16 nodes x R rows each; the A operand is
+// staged in one orientation ([G][R] rows of [16 jl][S]) whichever side of the diagonal the block lies on, and t is
+// read at the start of a step (no copy of it kept for the next).
+constexpr int GBS_NODES = 64;   // nodes per workgroup
+template <int D, int S, int R, bool BLK>
+__global__ __launch_bounds__(256, 2) void backward_small_kernel(int64_t N, int nC, float scale,
+                                                                const float* __restrict__ g,
+                                                                const float* __restrict__ t,
+                                                                const _Float16* __restrict__ Wb2,
+                                                                const float* __restrict__ winv,
+                                                                float* __restrict__ dt) {
+  constexpr int G = 16 / R;
+  constexpr int KS = S / 32;
+  constexpr int RS = S + 8, AS = 16 * RS + 8, PS = 16 * AS;   // as above: rows (column block, il) of [jl][o]
+  constexpr int PW = 2 * 256 * S / 8 / 256;                   // 16-byte pieces of a step per thread
+  __shared__ __align__(16) _Float16 wl[2 * PS];
+  const int nb = nC / 16, np = n_pairs(nb);
+  const int I = blockIdx.x / G, il0 = (blockIdx.x % G) * R;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int r = lane & 15, q = lane >> 4;
+  const int64_t n = (int64_t)blockIdx.y * GBS_NODES + wave * 16 + r;
+  const bool valid = n < N;
+  const int64_t nl = valid ? n : 0;   // rows past N read node 0; their results are not stored
+  const bool idle = (int64_t)blockIdx.y * GBS_NODES + wave * 16 >= N;   // wave-uniform: stages only
+  const f4 zero = {0.f, 0.f, 0.f, 0.f};
+  float gv[KS][8];
+  float gmax = 0.f;
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    const f4 x0 = valid ? ld4(g + n * S + 32 * ks + 8 * q) : zero;
+    const f4 x1 = valid ? ld4(g + n * S + 32 * ks + 8 * q + 4) : zero;
+    gv[ks][0] = x0.x; gv[ks][1] = x0.y; gv[ks][2] = x0.z; gv[ks][3] = x0.w;
+    gv[ks][4] = x1.x; gv[ks][5] = x1.y; gv[ks][6] = x1.z; gv[ks][7] = x1.w;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) gmax = fmaxf(gmax, fabsf(gv[ks][j]));
+  }
+  gmax = fmaxf(gmax, __shfl_xor(gmax, 16, 64));
+  gmax = fmaxf(gmax, __shfl_xor(gmax, 32, 64));
+  const float sg = pow2_scale(gmax);
+  h8 gh[KS], gl[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) split2h(gv[ks], sg, gh[ks], gl[ks]);
+  float acc[R][D];
+#pragma unroll
+  for (int i = 0; i < R; ++i)
+#pragma unroll
+    for (int m = 0; m < D; ++m) acc[i][m] = 0.f;
+  f4 pw[PW];
+  const int64_t plane = (int64_t)np * 256 * S;
+  // piece idx of a step: plane, staged row (column block J0 + row / R, il0 + row % R), jl, 8 outputs
+  auto fetch = [&](int J0) {
+#pragma unroll
+    for (int i = 0; i < PW; ++i) {
+      const int idx = threadIdx.x + 256 * i;
+      const int pl = idx / (32 * S), rem = idx - pl * (32 * S);
+      const int row = rem / (2 * S), jl = (rem / (S / 8)) % 16, o8 = rem % (S / 8);
+      const int J = min(J0 + row / R, nb - 1), il = il0 + row % R;
+      const int pr = (I <= J) ? pair_index(I, J, nb) : pair_index(J, I, nb);
+      const int ab = (I <= J) ? il * 16 + jl : jl * 16 + il;
+      pw[i] = *reinterpret_cast<const f4*>(Wb2 + pl * plane + ((int64_t)pr * 256 + ab) * S + 8 * o8);
+    }
+  };
+  fetch(0);
+  for (int J0 = 0; J0 < nb; J0 += G) {
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < PW; ++i) {
+      const int idx = threadIdx.x + 256 * i;
+      const int pl = idx / (32 * S), rem = idx - pl * (32 * S);
+      const int row = rem / (2 * S), jl = (rem / (S / 8)) % 16, o8 = rem % (S / 8);
+      *reinterpret_cast<f4*>(&wl[pl * PS + row * AS + jl * RS + 8 * o8]) = pw[i];
+    }
+    __syncthreads();
+    if (J0 + G < nb) fetch(J0 + G);
+    __builtin_amdgcn_sched_barrier(0);
+    if (idle) continue;
+    // the step's t at once, or for D 7 and 9 (registers) a column block ahead
+    constexpr int NTC = D <= 5 ? G : 2;
+    f4 tc[NTC][D];
+    auto load_t = [&](int c) {
+#pragma unroll
+      for (int m = 0; m < D; ++m)
+        tc[c % NTC][m] = ld4(tq4<BLK>(t, N, D, nC, nl, m, min(J0 + c, nb - 1) * 16 + 4 * q));
+    };
+#pragma unroll
+    for (int c = 0; c < (D <= 5 ? G : 1); ++c) load_t(c);
+#pragma unroll
+    for (int c = 0; c < G; ++c) {
+      if constexpr (D > 5) {
+        if (c + 1 < G) load_t(c + 1);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (J0 + c >= nb) break;
+#pragma unroll
+      for (int i = 0; i < R; ++i) {
+        f4 dd = zero;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+          const int off = (c * R + i) * AS + r * RS + 32 * ks + 8 * q;
+          const h8 oh = *reinterpret_cast<const h8*>(&wl[off]);
+          const h8 ol = *reinterpret_cast<const h8*>(&wl[PS + off]);
+          dd = mfma_x3(oh, ol, gh[ks], gl[ks], dd);
+        }
+#pragma unroll
+        for (int m = 0; m < D; ++m)
+#pragma unroll
+          for (int k = 0; k < 4; ++k) acc[i][m] = fmaf(dd[k], tc[c % NTC][m][k], acc[i][m]);
+      }
+    }
+  }
+  const float f = scale * winv[0] / sg;   // sg is a power of two: exact
+#pragma unroll
+  for (int i = 0; i < R; ++i)
+#pragma unroll
+    for (int m = 0; m < D; ++m) {
+      float v = acc[i][m];
+      v += __shfl_xor(v, 16, 64);
+      v += __shfl_xor(v, 32, 64);
+      if (valid && q == (i & 3)) dt[(n * D + m) * nC + I * 16 + il0 + i] = v * f;
+    }
+}
+
 int check_dims(int64_t N, int32_t D, int32_t nC, int32_t S, const char* who) {
   if (N < 0 || N >= (1LL << 31) || nC < 16 || nC % 16 != 0 || nC > 16 * 64 || !(S == 32 || S == 64) ||
       !(D == 1 || D == 3 || D == 5 || D == 7 || D == 9)) {
@@ -739,6 +864,12 @@ int forward_s(int64_t N, int D, int nC, float scale, const float* t, const float
 
 // largest D whose backward has the registers for the operand pipeline (at D 9 it spills)
 constexpr int GB_PIPE_DMAX = 7;
+// (64-node tile, row block) pairs up to which the small kernel, with four workgroups a pair, is the faster one.
+// nC 192, us, large / small, D 1, 3, 5 | 7, 9: 32 nodes (12 pairs) 37 / 12, 36 / 13, 41 / 15 | 33 / 15, 40 / 17;
+// 512 nodes (96) 39 / 17, 38 / 19, 44 / 24 | 36 / 26, 44 / 31; 1,000 nodes (192) 39 / 26, 39 / 33, 46 / 42 | 38 / 43,
+// 47 / 51; 2,000 nodes (384) 41 / 46, 41 / 55, 48 / 70.  nC 384, 256 nodes (96): 75 / 30, 73 / 34, 84 / 41 | 67 / 43,
+// 80 / 50.  The wide D turn earlier: the large kernel takes 64 nodes a workgroup for them as well.
+constexpr int64_t GBS_UNITS = 192, GBS_UNITS_WIDE = 128;
 
 template <int S, bool BLK>
 int backward_s(int64_t N, int D, int nC, float scale, const float* g, const float* t, const float* Wb, float* dt,
@@ -750,6 +881,22 @@ int backward_s(int64_t N, int D, int nC, float scale, const float* g, const floa
   const _Float16* Wb2 = reinterpret_cast<const _Float16*>(Wb + (int64_t)n_pairs(nC / 16) * 256 * S);
   const float* winv = Wb + (int64_t)n_pairs(nC / 16) * 512 * S;
   LaunchTimer tm("gram_backward", st);
+  const int64_t stiles = (N + GBS_NODES - 1) / GBS_NODES;
+  if (stiles * (nC / 16) <= (D <= 5 ? GBS_UNITS : GBS_UNITS_WIDE)) {
+    constexpr int R = 4;   // rows a workgroup (8 rows and two column blocks a step measured no gain at D 7 and 9)
+#define FSC_GBS(DD)                                                                                                  \
+  backward_small_kernel<DD, S, R, BLK><<<dim3((unsigned)(nC / 16 * (16 / R)), (unsigned)stiles), 256, 0, st>>>(      \
+      N, nC, scale, g, t, Wb2, winv, dt)
+    switch (D) {
+      case 1: FSC_GBS(1); break;
+      case 3: FSC_GBS(3); break;
+      case 5: FSC_GBS(5); break;
+      case 7: FSC_GBS(7); break;
+      default: FSC_GBS(9); break;
+    }
+#undef FSC_GBS
+    return check_launch("gram backward") ? 2 : 0;
+  }
 #define FSC_GBB(DD) \
   backward_h16_kernel<DD, S, (DD <= 5 ? 16 : 8), (DD > 1 && DD <= GB_PIPE_DMAX), BLK><<<grid, 512, 0, st>>>(N, nC, scale, \
                                                                                                     g, t, Wb2, \

@@ -48,6 +48,15 @@ def test_gram_bilinear_matches_reference(N, D, nC, S):
     assert rel_inf(gt, gref) < TOL
 
 
+# backward for few nodes (4 rows and 4 column blocks a step): node-tile edges at 64, column blocks not a multiple of
+# 4, the last sizes it takes (192 node tiles x row blocks, 128 at D 7 and 9) and the first of the large kernel
+@pytest.mark.parametrize("N,D,nC,S", [(64, 5, 96, 32), (65, 7, 112, 64), (129, 9, 208, 64), (63, 1, 80, 32),
+                                      (1024, 3, 192, 32), (1025, 3, 192, 32), (705, 1, 272, 64), (512, 7, 256, 32),
+                                      (513, 7, 256, 32), (460, 9, 272, 64), (1000, 5, 208, 64)])
+def test_gram_bilinear_backward_at_the_kernel_switch(N, D, nC, S):
+    test_gram_bilinear_matches_reference(N, D, nC, S)
+
+
 def test_gram_bilinear_strided_input_and_empty():
     """A transposed (non-contiguous) view gives the same result; zero nodes give an empty output."""
     from fsctep_amd import readout_ops  # noqa: F401
