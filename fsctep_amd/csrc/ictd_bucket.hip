@@ -11,10 +11,11 @@
 // g [B][P], out [B][O][K].
 //
 // The projections contract over at most 9 x 9 components and run on the VALU, one wave per batch
-// element with the factor ub[m][pk] = sum_n v[n] U[m*m2+n][pk] formed once per element in LDS.  The
-// channel mixes are GEMMs over (b, k) rows and run on v_mfma_f32_16x16x4_f32 (fp32) or
-// v_mfma_f64_16x16x4_f64 (fp64; MI355X runs fp64 matrix and vector FMAs at the same peak, the MFMA form keeps
-// the operand reuse of the tile).  Every kernel is templated on the element type T.  Every kernel writes or,
+// element with the factor ub[m][pk] = sum_n v[n] U[m*m2+n][pk] formed once per element in LDS (the
+// gradient of v alone on the matrix cores).  The channel mixes are GEMMs over (b, k) rows: fp64 on
+// v_mfma_f64_16x16x4_f64 (MI355X runs fp64 matrix and vector FMAs at the same peak, the MFMA form keeps the
+// operand reuse of the tile); fp32 up to 128 channels with the weights resident in LDS and split-fp16
+// products, otherwise, and for the weight gradient, on v_mfma_f32_16x16x4_f32.  Every kernel writes or,
 // with `acc`, adds to its output, so the double-backward sums of the reference (csrc/ictd_tp_cuda.cu:528-533,
 // 796-802) are the same kernels run two or three times.  Sums over the batch (the gradients of U and W)
 // go through per-block partial sums and a reduction in a fixed order: results are deterministic.
