@@ -267,8 +267,9 @@ __global__ __launch_bounds__(256) void fill_kernel(Walk w, const int32_t* __rest
   const int lane = threadIdx.x & 63;
   const int64_t j = w.cell_atoms[p];
   const int64_t beg = dst_ptr[j], end = dst_ptr[j + 1] < E ? dst_ptr[j + 1] : E;
+  if (end <= beg) return;   // no neighbours, or a segment past a caller's E: the accesses below take deg > 0
   const int32_t deg = (int32_t)(end - beg);
-  // the counts came from the same walk, so rank < deg always holds: kept as a bound
+  // the counts came from the same walk, so rank < deg holds unless E cuts the segment: kept as a bound
   if (deg <= KEY_CAP && w.N < (int64_t)(UINT32_MAX / KEY_IMAGES)) {
     uint32_t* mine = reinterpret_cast<uint32_t*>(lkeys[wave]);
     if (lane < 4 && (deg & ~3) + lane < KEY_CAP) mine[(deg & ~3) + lane] = UINT32_MAX;

@@ -4,6 +4,7 @@ numpy statement of the reference semantics (utils/graph_utils.py:192-257: every 
 periodic axes, |pos[j] + s @ cell - pos[i]| < r, no self pair at s = 0).  Integer output: bit-exact, in
 the same receiver-sorted order (then by source and image)."""
 
+import ctypes
 import time
 
 import numpy as np
@@ -130,3 +131,33 @@ def test_receivers_around_the_key_capacity(n, r):
     _equal(got, _brute(pos, cell, r, (0, 0, 0)), n)
     deg = np.diff(got[3])
     assert deg.max() == n - 1 if r > 8.7 else (deg.max() > 512 and deg.min() < 512)
+
+
+def test_fill_stays_within_a_smaller_edge_count():
+    """fsc_neighbor_fill with fewer edges than the list has: receivers before the cut are whole, nothing is written
+    at or past it (receivers wholly past it have no room at all), also where more than 512 keys are ranked."""
+    from fsctep_amd import _lib
+    for n, side, r in ((70, 5.0, 9.0), (530, 5.0, 9.0), (90, 12.0, 4.0)):
+        pos = torch.tensor(np.random.default_rng(n).uniform(0.0, side, (n, 3)), device=DEV)
+        cell = torch.eye(3, dtype=torch.float64, device=DEV) * 100.0
+        want = _gpu(pos.cpu().numpy(), cell.cpu().numpy(), r, pbc=False)
+        ws_n = ctypes.c_int64()
+        _lib.call("fsc_neighbor_workspace", n, ctypes.byref(ws_n))
+        ws = torch.empty(ws_n.value, dtype=torch.int32, device=DEV)
+        dst_ptr = torch.empty(n + 1, dtype=torch.int32, device=DEV)
+        pbc, st = (ctypes.c_int32 * 3)(0, 0, 0), torch.cuda.current_stream().cuda_stream
+        _lib.call("fsc_neighbor_count", n, pos.data_ptr(), cell.data_ptr(), pbc, r, dst_ptr.data_ptr(), ws.data_ptr(), st)
+        ptr = dst_ptr.cpu().numpy()
+        E = int(ptr[n])
+        np.testing.assert_array_equal(ptr, want[3])
+        for cut in (1, int(ptr[3]), int(ptr[n // 2]) + 1, E - 1, E):
+            src = torch.full((E + 1024,), -7, dtype=torch.int64, device=DEV)
+            dst, sh = src.clone(), torch.full((E + 1024, 3), -7.0, dtype=torch.float64, device=DEV)
+            fill = torch.empty(3 * E, dtype=torch.int32, device=DEV)
+            _lib.call("fsc_neighbor_fill", n, cut, pos.data_ptr(), cell.data_ptr(), pbc, r, dst_ptr.data_ptr(),
+                      ws.data_ptr(), fill.data_ptr(), src.data_ptr(), dst.data_ptr(), sh.data_ptr(), st)
+            whole = int(ptr[np.searchsorted(ptr, cut, side="right") - 1])   # end of the last whole segment
+            for got, ref in zip((src, dst, sh), want):
+                got = got.cpu().numpy()
+                np.testing.assert_array_equal(got[:whole], ref[:whole])
+                assert (got[cut:] == -7).all()
