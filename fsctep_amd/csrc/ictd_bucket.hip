@@ -1013,12 +1013,15 @@ __global__ __launch_bounds__(256, 3) void mix32_tw_kernel(Dims d, const float* _
 // ---------------------------------------------------------------- channel mix, fp32, whole weight matrix resident
 // For at most 16 T input and output channels (T 2, 4, 8) one path's weight matrix fits in LDS (70 KB at 128
 // channels, two blocks a CU): it is staged once a block, and the four waves then walk row tiles of their own with
-// no barrier, the next tile's rows in flight during the products.  The products are split-fp16 (common.h): the matrix
-// is scaled by one power of two and staged as two fp16 planes, each row by the power of two of its own largest value
-// (both undone on the result), 3 MFMAs of 16 cycles a 32-deep step against 8 of 32 on the fp32 MFMA, which bound the
+// no barrier, the next tile's rows in flight during the products.  The products are split-fp16 (common.h): each column
+// of the product (an output channel's weights, or an input channel's in the gradients) is scaled by the power of two of
+// its own largest weight and staged as two fp16 planes, each row by the power of two of its own largest value (both
+// undone on the result), 3 MFMAs of 16 cycles a 32-deep step against 8 of 32 on the fp32 MFMA, which bound the
 // fp32 form of these kernels.  Error against 64 bits, 3,011 elements, outputs / gradients of the
-// gates: 1.5e-7 / 2.5e-7 at 128 channels, 1.1e-7 / 1.9e-7 at 32 (fp32 MFMA: 2.1e-7 / 2.9e-7, 1.2e-7 / 3.2e-7); a row
-// or matrix with a non-finite entry gives non-finite results and leaves the other rows' alone.
+// gates: 1.5e-7 / 2.5e-7 at 128 channels, 1.1e-7 / 1.9e-7 at 32 (fp32 MFMA: 2.1e-7 / 2.9e-7, 1.2e-7 / 3.2e-7), whatever
+// the rows' and the channels' magnitudes (one scale for the whole matrix left a channel 1e-10 below the largest with
+// 4e-2 of error); within one row or channel an entry keeps 2^-39 of the largest.  A row or channel with a non-finite
+// entry gives non-finite results and leaves the others' alone.
 // A tile is EB = 32 / K whole batch elements (row e K + k), so that a tile's outputs are contiguous.
 // 60,011 elements, K 7, 128 x 128, sliced kernels / resident with fp32 products / this: forward 260 / 214 / 118 us,
 // gate gradient 272 / 210 / 165, input gradient 171 + 5 / 190 / 168 (the last two read go in 4-byte pieces, element
@@ -1037,37 +1040,105 @@ __device__ __forceinline__ TileRow tile_row(int rho, int K, uint32_t mg, int EB)
 
 __device__ __forceinline__ float finite_abs(float v) { return fabsf(v) <= 3.402823466e38f ? fabsf(v) : 0.f; }
 
-// The matrix W [O][I] in LDS as the fp16 planes of W sw, zero beyond its size: ws[plane][o][i], or transposed (TRANS)
-// with column i of the product in row 16 (i % T) + i / T, so that a lane's T tiles are T consecutive columns.
-// sw is the power of two of the largest finite |W|; returns 1/sw.  Ends with a barrier.
+// k with max |x| 2^k in [2^13, 2^14) for the largest finite |x| of a row or column (0 where that is 0), at most 127:
+// below 2^-113 the scaled values are multiples of 2^-22 all the same, so nothing is lost.
+__device__ __forceinline__ int split_exponent(float mx) {
+  if (!(mx > 0.f)) return 0;
+  int e;
+  frexpf(mx, &e);   // mx = f 2^e, f in [0.5, 1)
+  return min(14 - e, 127);
+}
+__device__ __forceinline__ float pow2_of(int k) { return __int_as_float((k + 127) << 23); }   // -126 <= k <= 127
+
+// The factor gate 2^e of a row of results as a float and, in e, the exponent left over, 0 unless it is beyond 2^+-60.
+// A result's factor is the product of a row's, a column's and a gate's, which taken together can leave the range where
+// the result does not; its sum of scaled products lies in 2^-48 .. 2^35, so the float may be applied first.
+__device__ __forceinline__ float row_factor(float gate, int& e) {
+  int eg;
+  const float m = frexpf(gate, &eg);
+  const int all = e + eg, part = min(max(all, -60), 60);
+  e = all - part;
+  return m * pow2_of(part);
+}
+
+// The largest v >= 0 of each group of G = 8, 16 or 32 consecutive lanes, in all of them, without LDS (shuffles for each
+// of a thread's 16 rows cost 3 us a launch at 128 channels).
+template <int CTRL>
+__device__ __forceinline__ float dpp_max(float v) {
+  return fmaxf(v, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, true)));
+}
+template <int G>
+__device__ __forceinline__ float group_max(float v) {
+  v = dpp_max<0xB1>(v);    // lanes 1 0 3 2 of each four
+  v = dpp_max<0x4E>(v);    // lanes 2 3 0 1
+  v = dpp_max<0x141>(v);   // mirrored eight
+  if constexpr (G >= 16) v = dpp_max<0x140>(v);   // mirrored sixteen
+  if constexpr (G >= 32) {   // rows 0 and 1, 2 and 3 of sixteen lanes
+    typedef unsigned u2 __attribute__((ext_vector_type(2)));
+    const unsigned x = __float_as_uint(v);
+    const u2 w = __builtin_bit_cast(u2, __builtin_amdgcn_permlane16_swap(x, x, false, false));
+    v = fmaxf(__uint_as_float(w.x), __uint_as_float(w.y));
+  }
+  return v;
+}
+
+// The matrix W [O][I] in LDS as two fp16 planes, zero beyond its size: ws[plane][o][i], or transposed (TRANS) with
+// column i of the product in row 16 (i % T) + i / T, so that a lane's T tiles are T consecutive columns.  Each column
+// of the product (row o, or column i, of W) is scaled by the power of two of its own largest finite entry; ex[row of
+// ws] is the exponent that undoes it.  Ends with a barrier.
 template <int T, bool TRANS>
-__device__ __forceinline__ float stage_matrix(const float* __restrict__ W, int O, int I,
-                                              _Float16 (&ws)[2][16 * T][16 * T + 8], float (&red)[4]) {
+__device__ __forceinline__ void stage_matrix(const float* __restrict__ W, int O, int I,
+                                             _Float16 (&ws)[2][16 * T][16 * T + 8], int (&ex)[16 * T],
+                                             float (&red)[TRANS ? 4 : 1][16 * T]) {
   typedef _Float16 h4 __attribute__((ext_vector_type(4)));
   constexpr int NP = T * T / 4;
+  const int i = 4 * (threadIdx.x % (4 * T));   // the thread's four columns; rows o of piece s below
+  auto row = [&](int s) { return (int)(threadIdx.x + 256 * s) / (4 * T); };
   f4 v[NP];
-  float mx = 0.f;
 #pragma unroll
-  for (int s = 0; s < NP; ++s) {
-    const int idx = threadIdx.x + 256 * s, o = idx / (4 * T), i = 4 * (idx % (4 * T));
-    v[s] = ld4(W + (o < O && i < I ? (int64_t)o * I + i : 0));
-  }
+  for (int s = 0; s < NP; ++s) v[s] = ld4(W + (row(s) < O && i < I ? (int64_t)row(s) * I + i : 0));
 #pragma unroll
   for (int s = 0; s < NP; ++s)
+    if (!(row(s) < O && i < I)) v[s] = f4{0.f, 0.f, 0.f, 0.f};
+  float sc[TRANS ? 4 : NP];   // the scale of column i + u (TRANS) or of row(s)
+  if constexpr (TRANS) {
+    float mx[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int u = 0; u < 4; ++u) mx = fmaxf(mx, finite_abs(v[s][u]));
-  for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
-  __syncthreads();
-  const float sw = pow2_scale(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
+    for (int u = 0; u < 4; ++u) {
+#pragma unroll
+      for (int s = 0; s < NP; ++s) mx[u] = fmaxf(mx[u], finite_abs(v[s][u]));
+#pragma unroll
+      for (int off = 32; off >= 4 * T; off >>= 1) mx[u] = fmaxf(mx[u], __shfl_xor(mx[u], off, 64));
+    }
+    if ((threadIdx.x & 63) < 4 * T) st4(&red[threadIdx.x >> 6][i], f4{mx[0], mx[1], mx[2], mx[3]});
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int k = split_exponent(fmaxf(fmaxf(red[0][i + u], red[1][i + u]), fmaxf(red[2][i + u], red[3][i + u])));
+      sc[u] = pow2_of(k);
+      if (threadIdx.x < 4 * T) ex[16 * ((i + u) % T) + (i + u) / T] = -k;
+    }
+  } else {
+    int ks[NP];
+#pragma unroll
+    for (int s = 0; s < NP; ++s) {   // 4 T consecutive lanes hold a row
+      const float m4 =
+          fmaxf(fmaxf(finite_abs(v[s][0]), finite_abs(v[s][1])), fmaxf(finite_abs(v[s][2]), finite_abs(v[s][3])));
+      ks[s] = split_exponent(group_max<4 * T>(m4));
+      sc[s] = pow2_of(ks[s]);
+    }
+    if (i == 0) {
+#pragma unroll
+      for (int s = 0; s < NP; ++s) ex[row(s)] = -ks[s];
+    }
+  }
 #pragma unroll
   for (int s = 0; s < NP; ++s) {
-    const int idx = threadIdx.x + 256 * s, o = idx / (4 * T), i = 4 * (idx % (4 * T));
-    const bool ok = o < O && i < I;
+    const int o = row(s);
     h4 h, l;
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const float x = ok ? v[s][u] * sw : 0.f;
+      const float x = v[s][u] * sc[TRANS ? u : s];
       h[u] = (_Float16)x;
       l[u] = (_Float16)(x - (float)h[u]);
     }
@@ -1083,7 +1154,6 @@ __device__ __forceinline__ float stage_matrix(const float* __restrict__ W, int O
     }
   }
   __syncthreads();
-  return 1.f / sw;
 }
 
 // MODE 0: out[b][o][k] (+)= g[b] sum_i y[b][k][i] W[o][i]  (one path; src = y)
@@ -1098,12 +1168,13 @@ __global__ __launch_bounds__(256, 2) void mix32_resident_kernel(Dims d, int EB, 
                                                                 int acc) {
   constexpr int BLD = 36, HS = T / 2;   // HS: 32-deep contraction steps
   __shared__ __align__(16) _Float16 ws[2][16 * T][16 * T + 8];
-  __shared__ float red[4];
+  __shared__ __align__(16) float red[MODE != 0 ? 4 : 1][16 * T];
+  __shared__ int ex[16 * T];   // undoes the scale of a column of the product
   __shared__ __align__(16) float tr[MODE == 2 ? 1 : 4][MODE == 0 ? 16 * BLD : 32];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, q = lane >> 4;
   const int K = d.K, P = d.P, I = d.I, O = d.O, p = MODE == 0 ? 0 : (int)blockIdx.y;
-  const float winv = stage_matrix<T, MODE != 0>(W + (int64_t)p * O * I, O, I, ws, red);
+  stage_matrix<T, MODE != 0>(W + (int64_t)p * O * I, O, I, ws, ex, red);
   const int nk = MODE != 0 ? O : I;                                   // contraction length
   const int64_t sstride = MODE != 0 ? (int64_t)O * K : (int64_t)K * I;   // an element of src
   const uint32_t mg = 65536u / (uint32_t)K + 1;
@@ -1133,9 +1204,9 @@ __global__ __launch_bounds__(256, 2) void mix32_resident_kernel(Dims d, int EB, 
   if (tile >= ntiles) return;   // no barrier follows
   request(tile);
   for (; tile < ntiles; tile += tstep) {
-    // the rows split, each by the power of two of its largest finite value (its values sit in four lanes); fr undoes
-    // the scales on the row's results and applies the gate
+    // the rows split, each by the power of two of its largest finite value (its values sit in four lanes); er undoes it
     h8 xh[2][HS], xl[2][HS];
+    int er[2];
     float fr[2];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
@@ -1148,15 +1219,16 @@ __global__ __launch_bounds__(256, 2) void mix32_resident_kernel(Dims d, int EB, 
       }
       mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
       mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-      const float sr = pow2_scale(mx);
+      const int kr = split_exponent(mx);
+      const float sr = pow2_of(kr);
 #pragma unroll
       for (int h = 0; h < HS; ++h) {
         const float v[8] = {a[t][2 * h][0],     a[t][2 * h][1],     a[t][2 * h][2],     a[t][2 * h][3],
                             a[t][2 * h + 1][0], a[t][2 * h + 1][1], a[t][2 * h + 1][2], a[t][2 * h + 1][3]};
         split2h(v, sr, xh[t][h], xl[t][h]);
       }
-      fr[t] = winv / sr;   // exact: powers of two
-      if constexpr (MODE == 0) fr[t] *= gt[t];
+      er[t] = -kr;
+      if constexpr (MODE == 0) fr[t] = row_factor(gt[t], er[t]);
     }
     __builtin_amdgcn_sched_barrier(0);
     request(std::min(tile + tstep, ntiles - 1));
@@ -1175,20 +1247,33 @@ __global__ __launch_bounds__(256, 2) void mix32_resident_kernel(Dims d, int EB, 
 #pragma unroll
         for (int t = 0; t < 2; ++t) accm[t][j] = mfma_x3(xh[t][h], xl[t][h], wh, wl, accm[t][j]);
       }
-    // result register jj of lane group q is row 4 q + jj of the tile: its factor is held by lane 4 q + jj
+    int ew[T];
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int jj = 0; jj < 4; ++jj) {
-        const float f = __shfl(fr[t], 4 * q + jj, 64);
-#pragma unroll
-        for (int j = 0; j < T; ++j) accm[t][j][jj] *= f;
-      }
+    for (int j = 0; j < T; ++j) ew[j] = ex[16 * j + r];
     const int64_t b0 = tile * EB;
     const int nel = (int)std::min<int64_t>(EB, d.B - b0);
     uint32_t mge = mg;
     asm volatile("" : "+s"(mge));   // row indices are formed anew for each tile, not held across the products
+    // result register jj of lane group q is row 4 q + jj of the tile: its exponent and gate are held by lane 4 q + jj
     if constexpr (MODE == 0) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) {
+          const float f = __shfl(fr[t], 4 * q + jj, 64);
+#pragma unroll
+          for (int j = 0; j < T; ++j) accm[t][j][jj] = ldexpf(accm[t][j][jj] * f, ew[j]);
+        }
+      if (__ballot(er[0] | er[1])) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int jj = 0; jj < 4; ++jj) {
+            const int e = __shfl(er[t], 4 * q + jj, 64);
+#pragma unroll
+            for (int j = 0; j < T; ++j) accm[t][j][jj] = ldexpf(accm[t][j][jj], e);
+          }
+      }
       // out[b][o][k] holds an element's rows side by side: 16 columns at a time turn through LDS and leave in runs
       // of 16 K floats an element (a store per register would write 4 bytes every 4 K)
       float* ob = dst + b0 * O * K;
@@ -1224,6 +1309,10 @@ __global__ __launch_bounds__(256, 2) void mix32_resident_kernel(Dims d, int EB, 
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int jj = 0; jj < 4; ++jj) {
+          // the row's exponent is undone on its sum (the row at most 1 until then): y W is in range where go W need
+          // not be
+#pragma unroll
+          for (int j = 0; j < T; ++j) accm[t][j][jj] = ldexpf(accm[t][j][jj], ew[j] - 14);
           const TileRow w = tile_row(16 * t + 4 * q + jj, K, mge, EB);
           const float* yp = y + (((b0 + (w.el < nel ? w.el : 0)) * P + p) * K + w.k) * I;
           float v = 0.f;
@@ -1243,7 +1332,7 @@ __global__ __launch_bounds__(256, 2) void mix32_resident_kernel(Dims d, int EB, 
               v += i < I ? accm[t][j][jj] * yv : 0.f;
             }
           }
-          rowsum[4 * t + jj] = v;
+          rowsum[4 * t + jj] = ldexpf(v, __shfl(er[t], 4 * q + jj, 64) + 14);
           if (jj & 1) __builtin_amdgcn_sched_barrier(0);   // two rows of y in flight, not all eight (registers)
         }
       // over the 16 column lanes by halving exchanges: lane bits 3, 2, 1 choose the half of the rows kept
@@ -1272,24 +1361,27 @@ __global__ __launch_bounds__(256, 2) void mix32_resident_kernel(Dims d, int EB, 
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int jj = 0; jj < 4; ++jj) {
+          const int e0 = __shfl(er[t], 4 * q + jj, 64);
           const TileRow w = tile_row(16 * t + 4 * q + jj, K, mge, EB);
           if (!w.ok || w.el >= nel) continue;
           const int64_t b = b0 + w.el;
-          const float gate = g[b * P + p];
+          int e = e0;
+          const float f = row_factor(g[b * P + p], e);
           float* o = dst + ((b * P + p) * K + w.k) * I + T * r;
           if constexpr (T >= 4) {
 #pragma unroll
             for (int hh = 0; hh < T / 4; ++hh)
               if (T * r + 4 * hh < I) {   // I % 4 == 0
-                f4 v = {accm[t][4 * hh][jj], accm[t][4 * hh + 1][jj], accm[t][4 * hh + 2][jj], accm[t][4 * hh + 3][jj]};
-                v = v * gate;
+                f4 v;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) v[u] = ldexpf(accm[t][4 * hh + u][jj] * f, e + ew[4 * hh + u]);
                 if (acc) v = ld4(o + 4 * hh) + v;
                 st4(o + 4 * hh, v);
               }
           } else {
 #pragma unroll
             for (int j = 0; j < T; ++j)
-              if (T * r + j < I) put(o + j, accm[t][j][jj] * gate, acc);
+              if (T * r + j < I) put(o + j, ldexpf(accm[t][j][jj] * f, e + ew[j]), acc);
           }
         }
     }

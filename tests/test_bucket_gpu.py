@@ -133,6 +133,49 @@ def test_mix_ops_rows_of_any_magnitude(C):
         assert float(((x - r)[keep].abs().reshape(B - 1, -1).amax(1) / scale).max()) < TOL
 
 
+def _by(err, ref, dims):
+    """Largest 2-norm relative error over the entries along the dimensions not in dims."""
+    return float((err.pow(2).sum(dims) / ref.pow(2).sum(dims)).max().sqrt())
+
+
+# O and I at a tile's width and below it (the three widths of the resident kernels), the forward and both gradients
+@pytest.mark.parametrize("C", [28, 32, 64, 100, 128])
+def test_mix_ops_channels_of_any_magnitude(C):
+    """Output channels and input channels whose weights span ten decades, and rows of one element that do, each keep
+    their own relative accuracy (their own scale): Gaussian rows and channels, so a channel's 2-norm error is a few
+    2^-24 of its 2-norm."""
+    E, B, K = ext(), 90, 5
+    rows = torch.logspace(-8, 8, K, dtype=torch.float64)[torch.randperm(K, generator=torch.Generator().manual_seed(C))]
+    y, g = rnd(B, 1, K, C, seed=1) * rows.view(1, 1, K, 1), rnd(B, 1, seed=2)
+    go, unit = rnd(B, C, K, seed=3) * rows, rnd(B, 1, K, C, seed=4)
+    for o_mag, i_mag in ((10, 0), (0, 10), (10, 10)):
+        w = rnd(1, C, C, seed=5) * torch.logspace(0, -o_mag, C, dtype=torch.float64).view(1, C, 1)
+        w = w * torch.logspace(-i_mag, 0, C, dtype=torch.float64).view(1, 1, C)
+        y, w, g, go, unit = (t.float().double() for t in (y, w, g, go, unit))
+        out, ref = E.mix_bucket_forward(gpu(y), gpu(w), gpu(g)).double().cpu(), BR.mix_forward(y, w, g)
+        assert _by(out - ref, ref, (0,)) < TOL                              # each output channel of each row k
+        got, ref = E.mix_bucket_transpose_y(gpu(go), gpu(w), gpu(g)).double().cpu(), BR.mix_transpose(go, y, w, g)[0]
+        assert _by((got - ref)[:, 0], ref[:, 0], (0,)) < TOL                # each input channel of each row k
+        got, ref = E.mix_bucket_transpose_g(gpu(go), gpu(unit), gpu(w)).double().cpu(), BR.mix_transpose(go, unit, w, g)[2]
+        assert _by(got - ref, ref, (0, 1)) < TOL
+
+
+def test_mix_ops_scales_that_leave_the_range_together():
+    """Results within float32's range whose row scale, channel scale and gate are not when multiplied by each other
+    first; rows below the smallest scale."""
+    E, B, K, C = ext(), 33, 3, 64
+    y, w, g, go = rnd(B, 1, K, C, seed=1), rnd(1, C, C, seed=2), rnd(B, 1, seed=3), rnd(B, C, K, seed=4)
+    for sy, sw, sg, sgo in ((1e25, 1e25, 1e-25, 1e5), (1e-35, 1e30, 1e10, 1e-36), (1e20, 1e-10, 1e5, 1e-30),
+                            (1e30, 1e-36, 1e-2, 1e25), (1e-37, 1.0, 1.0, 1e-37)):
+        yy, ww, gg, oo = ((t * s).float().double() for t, s in ((y, sy), (w, sw), (g, sg), (go, sgo)))
+        ty, _, tg = BR.mix_transpose(oo, yy, ww, gg)
+        for name, got, ref in (("out", E.mix_bucket_forward(gpu(yy), gpu(ww), gpu(gg)), BR.mix_forward(yy, ww, gg)),
+                               ("y", E.mix_bucket_transpose_y(gpu(oo), gpu(ww), gpu(gg)), ty),
+                               ("g", E.mix_bucket_transpose_g(gpu(oo), gpu(yy), gpu(ww)), tg)):
+            if 1e-36 < float(ref.norm()) and float(ref.abs().max()) < 1e38:
+                assert _by(got.double().cpu() - ref, ref, tuple(range(ref.dim()))) < TOL, (name, sy, sw, sg, sgo)
+
+
 @pytest.mark.parametrize("case", [(5, 16, 9, 9, 1, 16), (9, 20, 3, 8, 1, 17), (7, 12, 9, 9, 4, 8), (6, 4, 1, 9, 3, 11),
                                   (3, 36, 5, 1, 7, 7), (8193, 8, 3, 5, 1, 64), (11, 18, 3, 3, 2, 3)])
 def test_direction_gradient_at_tile_edges(case):
