@@ -1068,8 +1068,8 @@ __global__ __launch_bounds__(256) void grad_absmax_kernel(const float* __restric
 //   dh[e][k]  = sum_{(slot,c)} dP[e][(slot,c)] S[m][(slot,c)][k]        A = dP rows, B = S      (K = 144)
 //   dS[k][col] = sum_e h[e][k] dP[e][col]                                A = h^T,     B = dP     (K = edges)
 // dP is held once, in LDS, as two fp16 planes of dP[e] * s_e, s_e the power of two of an upper bound of the
-// edge's row: |dP| <= 3 max|g| (|n| = 1: |g1.n|, |(g2 n)_i| <= sqrt 3 max|g|, |n.g2.n| <= 3 max|g|), from the
-// receiver's max |G| (grad_absmax_kernel).  The dh product undoes s_e per row; the dS product, whose K runs
+// edge's row: |dP| <= 3 max|g| max(1, |n|^2) (|g1.n|, |(g2 n)_i| <= sqrt 3 |n| max|g|, |n.g2.n| <= 3 |n|^2 max|g|;
+// directions need not be unit vectors), from the receiver's max |G| (grad_absmax_kernel).  The dh product undoes s_e per row; the dS product, whose K runs
 // over edges, takes h[e][k] / s_e as its A operand (exact: powers of two), scaled per k by the power of two of
 // that column's max, so the sum over edges needs no rescaling.  S is scaled per (chunk, k) by its own max and
 // each chunk's dh product is undone and added to the fp32 dh separately.  BF16S (the bf16 variant): S is held in
@@ -1165,15 +1165,17 @@ __global__ __launch_bounds__(256, 4) void edge_message_grad_h16_kernel(
       const int32_t d = edge_dst[id];
       eids[e] = id;
       dsts[e] = d;
-      const float se = pow2_scale(3.f * gmax[d] * scale);
-      esc[e] = se;
-      einv[e] = 1.f / se;
+      float nn = 0.f;
 #pragma unroll
       for (int k = 0; k < 3; ++k) {
         const float v = nvec[3 * (int64_t)id + k];
+        nn += v * v;
         ns[e][k] = (e < cnt) ? v : 0.f;
         dnacc[e][k] = 0.f;
       }
+      const float se = pow2_scale(3.f * gmax[d] * scale * fmaxf(nn, 1.f));
+      esc[e] = se;
+      einv[e] = 1.f / se;
     }
     __syncthreads();
     // A operand of the dS product for the whole edge block: lane (r, q) of wave w holds h[e][k] / s_e

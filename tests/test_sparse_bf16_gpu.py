@@ -53,6 +53,43 @@ def test_bf16_conv2_op_against_oracle(C):
     assert rel_inf(res[0][0], ref) < 1e-5                 # and the default path is the fp32-accurate one
 
 
+@pytest.mark.parametrize("prec", [0, 1])
+def test_directions_of_any_length(prec):
+    """The op takes any direction vectors: lengths from 0 to 50 (dP grows with the length's square), the default path
+    to 1e-5 and the bf16 variant to the bf16 bound of every output, edges of each decade of length by themselves too
+    (the gradient of a short direction is linear in the receiver gradient, that of a long one grows with it)."""
+    from fsctep_amd import ops
+    from fsctep_amd.graph import prepare_graph
+    from test_sparse_gpu import _graph_with_edge_cases
+    torch.manual_seed(5)
+    C, N = 32, 40
+    src, dst = _graph_with_edge_cases(N, 400, 9)
+    E = src.shape[0]
+    length = torch.logspace(-2, 1.7, E, dtype=torch.float64)[torch.randperm(E)]
+    length[:5] = 0.0
+    v = torch.randn(E, 3, dtype=torch.float64)
+    n = v / v.norm(dim=1, keepdim=True) * length.unsqueeze(1)
+    x, h = torch.randn(N, 13, C, dtype=torch.float64), torch.randn(E, 64, dtype=torch.float64)
+    L, b = torch.randn(6 * C * C, 64, dtype=torch.float64) / 8, torch.randn(6 * C * C, dtype=torch.float64) * 0.1
+    order = torch.argsort(dst, stable=True)
+    xo, ho, no = (t.clone().requires_grad_(True) for t in (x, h[order], n[order]))
+    ref = oracle_conv2(xo, ho, no, L, b, src[order], dst[order], N, 1.0 / (E / N))
+    G = torch.randn_like(ref)
+    gx, gh, gn = torch.autograd.grad((ref * G).sum(), (xo, ho, no))
+    gr = prepare_graph(src.to(DEV), dst.to(DEV), torch.zeros(E, 3, device=DEV), N)
+    bk1, bk6 = torch.ops.fsctep.sparse_prepare_weights(L.float().to(DEV), b.float().to(DEV), C)
+    xd, hd, nd = (t.float().to(DEV).requires_grad_(True) for t in (x, h[order], n[order]))
+    out = ops.sparse_conv_apply(xd, hd, nd, bk1, bk6, gr, precision=prec)
+    dx, dh, dn = torch.autograd.grad(out, (xd, hd, nd), G.float().to(DEV))
+    tol = TOL_BF16 if prec else 1e-5
+    assert max(rel_inf(a, r) for a, r in zip((out.detach(), dx, dh, dn), (ref, gx, gh, gn))) < tol
+    ls = length[order]
+    for lo, hi in ((-1.0, 0.1), (0.1, 1.0), (1.0, 4.0), (4.0, 60.0)):
+        m = (ls >= lo) & (ls < hi)
+        assert m.any()
+        assert rel_inf(dh.cpu()[m], gh[m]) < tol and rel_inf(dn.cpu()[m], gn[m]) < tol
+
+
 def test_bf16_model_against_fp32_path_and_deterministic():
     import bench
     from fsctep_amd.sparse import energy_and_forces
