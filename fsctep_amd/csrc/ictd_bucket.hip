@@ -90,6 +90,12 @@ __device__ __forceinline__ void form_ub(const Dims& d, int PK, const T* __restri
   }
 }
 
+// Sixteen bytes at any float's address (one access all the same): the operations take operands and outputs of any
+// alignment, views at an odd offset among them.
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ f4 ld4u(const float* p) { return *reinterpret_cast<const f4u*>(p); }
+__device__ __forceinline__ void st4u(float* p, const f4& v) { *reinterpret_cast<f4u*>(p) = v; }
+
 template <typename T>
 __device__ __forceinline__ void put(T* p, T v, int acc) { *p = acc ? *p + v : v; }
 
@@ -674,7 +680,7 @@ struct WSlice {
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
       const int c = c0 + (threadIdx.x >> 3) + 32 * s, k = k0 + 4 * (threadIdx.x & 7);
-      v[s] = ld4(w + (inside(s, ncol, nk, c0, k0) ? (int64_t)c * nk + k : 0));
+      v[s] = ld4u(w + (inside(s, ncol, nk, c0, k0) ? (int64_t)c * nk + k : 0));
     }
   }
   __device__ __forceinline__ f4 piece(int s, int ncol, int nk, int c0, int k0) const {
@@ -745,7 +751,7 @@ __global__ __launch_bounds__(256, 3) void mix32_kernel(Dims d, const float* __re
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           const int i = s * KS + 16 * h + 4 * q;
-          an[h][t] = ld4(y + yb[t] + (int64_t)p * K * I + (i < I ? i : 0));
+          an[h][t] = ld4u(y + yb[t] + (int64_t)p * K * I + (i < I ? i : 0));
         }
       }
     };
@@ -912,8 +918,8 @@ __global__ __launch_bounds__(256, 3) void mix32_ty_kernel(Dims d, const float* _
         if (i0 + 8 * r + 4 * hh < I) {   // I % 4 == 0
           f4 v = {accm[t][4 * hh][jj], accm[t][4 * hh + 1][jj], accm[t][4 * hh + 2][jj], accm[t][4 * hh + 3][jj]};
           v = v * gate;
-          if (acc) v = ld4(o + 4 * hh) + v;
-          st4(o + 4 * hh, v);
+          if (acc) v = ld4u(o + 4 * hh) + v;
+          st4u(o + 4 * hh, v);
         }
     }
 }
@@ -956,7 +962,7 @@ __global__ __launch_bounds__(256, 3) void mix32_tw_kernel(Dims d, const float* _
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const uint32_t row = std::min(rr + yrow + (64 / T) * u, r1 - 1), b = row / (uint32_t)K;
-      yn[u] = ld4(y + (((int64_t)b * P + p) * K + (row - b * K)) * I + (yok ? i0 + ycol : 0));
+      yn[u] = ld4u(y + (((int64_t)b * P + p) * K + (row - b * K)) * I + (yok ? i0 + ycol : 0));
     }
     // go: 16 rows of one column; the element and row in it advance without divisions
     const uint32_t first = std::min(rr + orow, r1 - 1);
@@ -1096,7 +1102,7 @@ __device__ __forceinline__ void stage_matrix(const float* __restrict__ W, int O,
   auto row = [&](int s) { return (int)(threadIdx.x + 256 * s) / (4 * T); };
   f4 v[NP];
 #pragma unroll
-  for (int s = 0; s < NP; ++s) v[s] = ld4(W + (row(s) < O && i < I ? (int64_t)row(s) * I + i : 0));
+  for (int s = 0; s < NP; ++s) v[s] = ld4u(W + (row(s) < O && i < I ? (int64_t)row(s) * I + i : 0));
 #pragma unroll
   for (int s = 0; s < NP; ++s)
     if (!(row(s) < O && i < I)) v[s] = f4{0.f, 0.f, 0.f, 0.f};
@@ -1195,7 +1201,7 @@ __global__ __launch_bounds__(256, 2) void mix32_resident_kernel(Dims d, int EB, 
 #pragma unroll
           for (int u = 0; u < 4; ++u) a[t][h][u] = sp[(int64_t)(kc + u) * K];
         } else {
-          a[t][h] = ld4(sp + kc);
+          a[t][h] = ld4u(sp + kc);
         }
       }
     }
@@ -1320,7 +1326,7 @@ __global__ __launch_bounds__(256, 2) void mix32_resident_kernel(Dims d, int EB, 
 #pragma unroll
             for (int hh = 0; hh < T / 4; ++hh) {
               const bool iv = T * r + 4 * hh < I;   // I % 4 == 0
-              const f4 yv = ld4(yp + (iv ? T * r + 4 * hh : 0));
+              const f4 yv = ld4u(yp + (iv ? T * r + 4 * hh : 0));
 #pragma unroll
               for (int u = 0; u < 4; ++u) v += iv ? accm[t][4 * hh + u][jj] * yv[u] : 0.f;
             }
@@ -1375,8 +1381,8 @@ __global__ __launch_bounds__(256, 2) void mix32_resident_kernel(Dims d, int EB, 
                 f4 v;
 #pragma unroll
                 for (int u = 0; u < 4; ++u) v[u] = ldexpf(accm[t][4 * hh + u][jj] * f, e + ew[4 * hh + u]);
-                if (acc) v = ld4(o + 4 * hh) + v;
-                st4(o + 4 * hh, v);
+                if (acc) v = ld4u(o + 4 * hh) + v;
+                st4u(o + 4 * hh, v);
               }
           } else {
 #pragma unroll

@@ -346,8 +346,8 @@ int fsc_ictd_conv1_backward(const FscIctdLayout* layout, int64_t n_nodes, int64_
  * Layouts: a [B][I][m1], v [B][1][m2], u [m1*m2][P*K], y [B][P][K][I], w [P][O][I], gates [B][P],
  * out [B][O][K].  accumulate != 0 adds to the output instead of overwriting it (the double-backward
  * sums).  Limits: m1, m2 <= 9, P*K <= 64 (projection; the U gradient also m1*m2*P*K <= 2048);
- * I, O multiples of 4 and K <= 128 (mix).  The U and W gradients sum over the batch through the
- * caller's workspace in a fixed order (deterministic). */
+ * I, O multiples of 4 and K <= 128 (mix).  Arrays need the alignment of their elements only.  The U and W
+ * gradients sum over the batch through the caller's workspace in a fixed order (deterministic). */
 /* project_bucket_forward (csrc/ictd_tp.cpp:140-176): y from a, v, u. */
 int fsc_bucket_project(int64_t B, int32_t I, int32_t m1, int32_t m2, int32_t P, int32_t K, const float* a,
                        const float* v, const float* u, float* y, int32_t accumulate, hipStream_t stream);

@@ -7,6 +7,7 @@ float64 (the reference's fp64 rtol, test/test_ictd_tp_backend.py:383-714).  Also
 table the ops reproduce the trunk's fully connected TP (oracle fctp); argument errors; an empty batch;
 bitwise-deterministic batch sums; the module passes the reference's availability probe."""
 
+import ctypes
 import sys
 
 import pytest
@@ -174,6 +175,48 @@ def test_mix_ops_scales_that_leave_the_range_together():
                                ("g", E.mix_bucket_transpose_g(gpu(oo), gpu(yy), gpu(ww)), tg)):
             if 1e-36 < float(ref.norm()) and float(ref.abs().max()) < 1e38:
                 assert _by(got.double().cpu() - ref, ref, tuple(range(ref.dim()))) < TOL, (name, sy, sw, sg, sgo)
+
+
+# each width of the resident kernels, the sliced kernels, several paths
+@pytest.mark.parametrize("case", [(70, 1, 3, 32, 20), (70, 2, 5, 64, 64), (70, 1, 7, 128, 100), (40, 2, 3, 132, 136),
+                                  (9, 1, 33, 64, 36)])
+def test_mix_ops_at_any_alignment(case):
+    """Operands one, two and three floats past a 16-byte boundary (views into a larger buffer), and outputs through the
+    C entry points at the same offsets: the aligned results, bit for bit."""
+    from fsctep_amd import _lib
+    B, P, K, I, O = case
+    E = ext()
+    y, w, g, go = (gpu(rnd(*s, seed=i)) for i, s in enumerate([(B, P, K, I), (P, O, I), (B, P), (B, O, K)]))
+
+    def shifted(t, off):
+        buf = torch.empty(t.numel() + 4, device=DEV)
+        v = buf[off:off + t.numel()].view(t.shape)
+        assert buf.data_ptr() % 16 == 0
+        return v.copy_(t)
+
+    def ops(y, w, g, go):
+        return [E.mix_bucket_forward(y, w, g), E.mix_bucket_transpose_y(go, w, g), E.mix_bucket_transpose_w(go, y, g),
+                E.mix_bucket_transpose_g(go, y, w)]
+
+    want = ops(y, w, g, go)
+    ws_n = ctypes.c_int64()
+    _lib.call("fsc_bucket_mix_workspace", B, P, K, I, O, ctypes.byref(ws_n))
+    ws = torch.empty(ws_n.value, device=DEV)
+    st = torch.cuda.current_stream().cuda_stream
+    for off in (1, 2, 3):
+        ys, wsh, gs, gos = (shifted(t, off) for t in (y, w, g, go))
+        for a, b in zip(ops(ys, wsh, gs, gos), want):
+            assert torch.equal(a, b)
+        outs = [shifted(torch.zeros_like(t), off) for t in want]
+        p = [t.data_ptr() for t in (ys, wsh, gs, gos)]
+        o = [t.data_ptr() for t in outs]
+        dims = (B, P, K, I, O)
+        _lib.call("fsc_bucket_mix", *dims, p[0], p[1], p[2], o[0], 0, st)
+        _lib.call("fsc_bucket_mix_transpose_y", *dims, p[3], p[1], p[2], o[1], 0, ws.data_ptr(), st)
+        _lib.call("fsc_bucket_mix_transpose_w", *dims, p[3], p[0], p[2], o[2], 0, ws.data_ptr(), st)
+        _lib.call("fsc_bucket_mix_transpose_g", *dims, p[3], p[0], p[1], o[3], 0, st)
+        for a, b in zip(outs, want):
+            assert torch.equal(a, b)
 
 
 @pytest.mark.parametrize("case", [(5, 16, 9, 9, 1, 16), (9, 20, 3, 8, 1, 17), (7, 12, 9, 9, 4, 8), (6, 4, 1, 9, 3, 11),
