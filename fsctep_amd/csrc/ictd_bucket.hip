@@ -40,6 +40,12 @@ struct Dims {
 
 typedef double d4 __attribute__((ext_vector_type(4)));
 
+// Sixteen bytes at any float's address (one access all the same): the operations take operands and outputs of any
+// alignment, views at an odd offset among them.
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ f4 ld4u(const float* p) { return *reinterpret_cast<const f4u*>(p); }
+__device__ __forceinline__ void st4u(float* p, const f4& v) { *reinterpret_cast<f4u*>(p) = v; }
+
 // One 16-deep K step of a 16 x 16 output tile for either element type.  Both MFMAs take lane l's operands
 // as A[l%16][l/16] and B[l/16][l%16]; their results differ in layout: register j of lane l holds
 // D[4*(l/16) + j][l%16] for v_mfma_f32_16x16x4_f32 and D[l/16 + 4*j][l%16] for v_mfma_f64_16x16x4_f64
@@ -51,7 +57,7 @@ struct Mma<float> {
   using V = f4;
   static __device__ __forceinline__ V zero() { return V{0.f, 0.f, 0.f, 0.f}; }
   static __device__ __forceinline__ V mma(const V& a, const V& b, V c) { return mfma_k16(a, b, c); }
-  static __device__ __forceinline__ V ld(const float* p) { return ld4(p); }
+  static __device__ __forceinline__ V ld(const float* p) { return ld4u(p); }
   static __device__ __forceinline__ int row(int q, int j) { return 4 * q + j; }
 };
 template <>
@@ -89,12 +95,6 @@ __device__ __forceinline__ void form_ub(const Dims& d, int PK, const T* __restri
     ub[idx] = m < d.m1 ? s : T(0);
   }
 }
-
-// Sixteen bytes at any float's address (one access all the same): the operations take operands and outputs of any
-// alignment, views at an odd offset among them.
-typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
-__device__ __forceinline__ f4 ld4u(const float* p) { return *reinterpret_cast<const f4u*>(p); }
-__device__ __forceinline__ void st4u(float* p, const f4& v) { *reinterpret_cast<f4u*>(p) = v; }
 
 template <typename T>
 __device__ __forceinline__ void put(T* p, T v, int acc) { *p = acc ? *p + v : v; }
@@ -377,8 +377,9 @@ __global__ __launch_bounds__(256) void sum_parts_kernel(int64_t n, int nparts, c
 }
 unsigned sum_parts_grid(int64_t n) { return (unsigned)std::min<int64_t>((n + 31) / 32, 4096); }
 
-// ---------------------------------------------------------------- channel mix (MFMA), fp64
-// Used for double, whose operands are twice as large; the fp32 forms are further down.
+// ---------------------------------------------------------------- channel mix (MFMA), every wave for itself
+// All of fp64, whose operands are twice as large; of fp32 the sizes that fill neither a slice nor the chip (mix_sliced
+// and the entry points), the other fp32 forms are further down.
 // Rows are the (b, k) pairs R = b*K + k.  A wave takes two 16-row tiles and eight 16-column tiles; lane
 // (r, q) of an MFMA supplies A[r][4q..4q+3] and B[4q..4q+3][r] for a 16-deep K step and ends with
 // D[4q + j][r] in result register j (common.h).
@@ -392,6 +393,9 @@ __global__ __launch_bounds__(256) void mix_kernel(Dims d, const T* __restrict__ 
                                                   T* __restrict__ out, int acc) {
   using M = Mma<T>;
   using V = typename M::V;
+  // fp32 requests the next K step's operands before the current products (two register sets); fp64,
+  // whose operand sets are twice as large, works one step at a time
+  constexpr bool PF = sizeof(T) == 4;
   __shared__ T rs[128];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, q = lane >> 4;
@@ -457,11 +461,27 @@ __global__ __launch_bounds__(256) void mix_kernel(Dims d, const T* __restrict__ 
         for (int j = 0; j < 8; ++j) accm[t][j] = M::mma(a, bw[j], accm[t][j]);
       }
     };
-    for (int st = 0; st < nst; ++st) {
-      V a0[2], b0[8];
-      T g0[2];
-      load(st, a0, g0, b0);
-      mma(a0, g0, b0);
+    if constexpr (PF) {
+      V a0[2], b0[8], a1[2], b1[8];
+      T g0[2], g1[2];
+      if (nst > 0) load(0, a0, g0, b0);
+      for (int st = 0; st < nst; st += 2) {
+        if (st + 1 < nst) load(st + 1, a1, g1, b1);
+        __builtin_amdgcn_sched_barrier(0);
+        mma(a0, g0, b0);
+        if (st + 1 < nst) {
+          if (st + 2 < nst) load(st + 2, a0, g0, b0);
+          __builtin_amdgcn_sched_barrier(0);
+          mma(a1, g1, b1);
+        }
+      }
+    } else {
+      for (int st = 0; st < nst; ++st) {
+        V a0[2], b0[8];
+        T g0[2];
+        load(st, a0, g0, b0);
+        mma(a0, g0, b0);
+      }
     }
 #pragma unroll
     for (int t = 0; t < 2; ++t)
@@ -796,10 +816,16 @@ __global__ __launch_bounds__(256, 3) void mix32_kernel(Dims d, const float* __re
         }
     } else {
       // out[b][o][k] holds an element's rows side by side: a store per register would write 4 bytes every 4K.
-      // 32 columns at a time pass through LDS, [column][row], and leave in runs of 32 K floats an element.
+      // 32 columns at a time pass through LDS, [column][row], and leave in runs of 32 K floats an element.  A
+      // thread's values are 256 apart in (element, column, k), reached by carries: dividing for each of them took
+      // 5 to 15 us of a launch.
       const uint32_t nrow = rend - rbeg, b0 = rbeg / (uint32_t)K, nb = (rend - 1) / (uint32_t)K - b0 + 1;
+      const uint32_t dc = 256u / (uint32_t)K, dk = 256u - dc * K;
+      const uint32_t c1 = threadIdx.x / (uint32_t)K, k1 = threadIdx.x - c1 * K;
 #pragma unroll
       for (int sl = 0; sl < 4; ++sl) {
+        const int oc = std::min(32, O - o0 - 32 * sl);   // columns of the slice
+        if (oc <= 0) break;                               // the same for every thread
         __syncthreads();
 #pragma unroll
         for (int t = 0; t < 2; ++t)
@@ -807,15 +833,17 @@ __global__ __launch_bounds__(256, 3) void mix32_kernel(Dims d, const float* __re
           for (int jh = 0; jh < 2; ++jh)
             st4(ws + (16 * jh + r) * OPAD + wave * 32 + 16 * t + 4 * q, accm[t][2 * sl + jh]);
         __syncthreads();
-        const int oc = std::min(32, O - o0 - 32 * sl);   // columns of the slice
-        if (oc > 0) {
-          const uint32_t run = (uint32_t)oc * K;
-          for (uint32_t idx = threadIdx.x; idx < nb * run; idx += 256) {
-            const uint32_t bi = idx / run, rem = idx - bi * run, c = rem / (uint32_t)K, k = rem - c * K;
-            const int32_t lr = (int32_t)((b0 + bi) * K + k - rbeg);
-            if (lr >= 0 && lr < (int32_t)nrow)
-              put(out + ((int64_t)(b0 + bi) * O + o0 + 32 * sl) * K + rem, ws[c * OPAD + lr], acc);
-          }
+        uint32_t bi = c1 >> 5, c = c1 & 31, k = k1;
+#pragma unroll 4
+        while (bi < nb) {
+          const int32_t lr = (int32_t)((b0 + bi) * K + k - rbeg);
+          if (lr >= 0 && lr < (int32_t)nrow && (int)c < oc)
+            put(out + ((int64_t)(b0 + bi) * O + o0 + 32 * sl + c) * K + k, ws[c * OPAD + lr], acc);
+          k += dk;
+          c += dc;
+          if (k >= (uint32_t)K) { k -= K; ++c; }
+          bi += c >> 5;
+          c &= 31;
         }
       }
     }
@@ -1424,6 +1452,12 @@ int resident_width(const Dims& d) {
   return c <= 32 ? 2 : c <= 64 ? 4 : 8;
 }
 
+// The forward slice by slice: enough workgroups that the slices' barriers are covered by other blocks, and channels
+// that leave less than half of the last 32-step slice empty.  Against every wave for itself (mix_kernel), us, three
+// paths: 128 channels, K 7, 55 workgroups 41 / 44, K 17, 133: 46 / 47, K 5, 391: 82 / 76, K 7, 547: 121 / 103; 144
+// channels, K 64, 1,000 workgroups: 161 / 175; 4 channels, K 7, 547: 19 / 25.
+bool mix_sliced(const Dims& d, int64_t workgroups) { return workgroups >= 320 && (d.I % 32 == 0 || d.I % 32 > 16); }
+
 template <int MODE>
 void launch_resident(const Dims& d, int t, const float* src, const float* w, const float* g, const float* y, float* dst,
                      int acc, hipStream_t st) {
@@ -1541,12 +1575,16 @@ int mix(int64_t B, int32_t P, int32_t K, int32_t I, int32_t O, const T* y, const
   const dim3 grid((unsigned)((B * K + 127) / 128), (unsigned)((O + 127) / 128));
   if constexpr (std::is_same_v<T, float>) {
     const int t = P == 1 ? resident_width(d) : 0;   // several paths add up in one product: slice by slice
-    if (t)
+    if (t) {
       launch_resident<0>(d, t, y, w, gates, nullptr, out, accumulate, st);
-    else
+      return check_launch("bucket mix") ? 2 : 0;
+    }
+    if (mix_sliced(d, (int64_t)grid.x * grid.y)) {
       mix32_kernel<false><<<grid, 256, 0, st>>>(d, y, w, gates, nullptr, out, accumulate);
-  } else
-    mix_kernel<T, false><<<grid, 256, 0, st>>>(d, y, w, gates, nullptr, out, accumulate);
+      return check_launch("bucket mix") ? 2 : 0;
+    }
+  }
+  mix_kernel<T, false><<<grid, 256, 0, st>>>(d, y, w, gates, nullptr, out, accumulate);
   return check_launch("bucket mix") ? 2 : 0;
 }
 
@@ -1559,12 +1597,18 @@ int mix_transpose_g(int64_t B, int32_t P, int32_t K, int32_t I, int32_t O, const
   const int BB = 128 / K;
   const dim3 grid((unsigned)((B + BB - 1) / BB), (unsigned)P);
   if constexpr (std::is_same_v<T, float>) {
-    if (const int t = resident_width(d))
+    if (const int t = resident_width(d)) {
       launch_resident<1>(d, t, grad_out, w, nullptr, y, grad_g, accumulate, st);
-    else
+      return check_launch("bucket mix_transpose_g") ? 2 : 0;
+    }
+    // at most half a slice of channels in a launch that does not fill the chip: every wave for itself (4 channels, K 17,
+    // one path, 1,000 elements in 143 workgroups: 8.3 us against 9.3; 10,000 elements: 39 against 28)
+    if (d.I > 16 || (int64_t)grid.x * grid.y > 160) {
       mix32_kernel<true><<<grid, 256, 0, st>>>(d, y, w, nullptr, grad_out, grad_g, accumulate);
-  } else
-    mix_kernel<T, true><<<grid, 256, 0, st>>>(d, y, w, nullptr, grad_out, grad_g, accumulate);
+      return check_launch("bucket mix_transpose_g") ? 2 : 0;
+    }
+  }
+  mix_kernel<T, true><<<grid, 256, 0, st>>>(d, y, w, nullptr, grad_out, grad_g, accumulate);
   return check_launch("bucket mix_transpose_g") ? 2 : 0;
 }
 
@@ -1609,10 +1653,14 @@ int mix_transpose_y(int64_t B, int32_t P, int32_t K, int32_t I, int32_t O, const
   transpose_w_kernel<T><<<(unsigned)std::min<int64_t>((nw + 255) / 256, 4096), 256, 0, st>>>(P, O, I, w, workspace);
   if (check_launch("bucket transpose_w")) return 2;
   const dim3 grid((unsigned)((B * K + 127) / 128), (unsigned)(P * ((I + 127) / 128)));
+  // at most 16 channels on both sides leave most of a slice and of a lane's eight columns empty: every wave for itself
+  // (16 channels, K 17, 20,000 elements: 35 us against 48)
   if constexpr (std::is_same_v<T, float>)
-    mix32_ty_kernel<<<grid, 256, 0, st>>>(d, grad_out, workspace, gates, grad_y, accumulate);
-  else
-    mix_ty_kernel<T><<<grid, 256, 0, st>>>(d, grad_out, workspace, gates, grad_y, accumulate);
+    if (std::max(I, O) > 16) {
+      mix32_ty_kernel<<<grid, 256, 0, st>>>(d, grad_out, workspace, gates, grad_y, accumulate);
+      return check_launch("bucket mix_transpose_y") ? 2 : 0;
+    }
+  mix_ty_kernel<T><<<grid, 256, 0, st>>>(d, grad_out, workspace, gates, grad_y, accumulate);
   return check_launch("bucket mix_transpose_y") ? 2 : 0;
 }
 
