@@ -253,10 +253,53 @@ __device__ __forceinline__ void write_edge(int64_t o, int64_t key, int64_t j, in
   edge_shifts[3 * o + 2] = (double)(code % 3 - 1);
 }
 
+// Ranks of the deg keys at `keys` (in memory, written by this wave), and their edges: a lane holds R keys, and all keys
+// pass by through the wave's part of LDS, as Key, CAP of them at a time (padded with the largest Key, compared 16 bytes
+// at a time).  Read past the L1, whose lines the segments of other receivers share.  3,000 receivers of 817 neighbours,
+// count and fill: 1.98 ms with a thread an edge over keys in memory, 2.23 ms with a wave a receiver over them, 0.47 ms
+// here; 2,000 of 920: 1.64, 2.38, 0.37 ms.
+template <typename Key, int R>
+__device__ __forceinline__ void rank_long(const int64_t* keys, int32_t deg, int lane, uint4* lds, int64_t beg, int64_t j,
+                                          int64_t* __restrict__ edge_src, int64_t* __restrict__ edge_dst,
+                                          double* __restrict__ edge_shifts) {
+  constexpr int CAP = KEY_CAP * 4 / (int)sizeof(Key), PER = 16 / (int)sizeof(Key);
+  Key* mine = reinterpret_cast<Key*>(lds);
+  const auto load = [&](int32_t t) {
+    return (Key)__hip_atomic_load(keys + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  for (int32_t t0 = 0; t0 < deg; t0 += 64 * R) {
+    Key key[R];
+    int32_t rank[R];
+#pragma unroll
+    for (int u = 0; u < R; ++u) {
+      const int32_t t = t0 + 64 * u + lane;
+      key[u] = load(t < deg ? t : deg - 1);
+      rank[u] = 0;
+    }
+    for (int32_t c0 = 0; c0 < deg; c0 += CAP) {
+      const int32_t n = deg - c0 < CAP ? deg - c0 : CAP;
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // the last keys are read
+#pragma unroll
+      for (int32_t i = lane; i < CAP; i += 64) mine[i] = i < n ? load(c0 + i) : ~Key(0);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      for (int32_t q = 0; PER * q < n; ++q) {
+        Key o[PER];
+        *reinterpret_cast<uint4*>(o) = lds[q];
+#pragma unroll
+        for (int u = 0; u < R; ++u)
+#pragma unroll
+          for (int v = 0; v < PER; ++v) rank[u] += o[v] < key[u];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < R; ++u)
+      if (t0 + 64 * u + lane < deg) write_edge(beg + rank[u], (int64_t)key[u], j, edge_src, edge_dst, edge_shifts);
+  }
+}
+
 // Keys of one receiver per wave, then each key's rank among them, which is its place in the receiver's
 // segment.  Up to KEY_CAP keys that fit 32 bits (159 million atoms) stay in LDS, padded with the largest key
-// so that they are compared four at a time; the others go through `keys` and are read back past the L1 (the
-// segments of other receivers share cache lines).
+// so that they are compared four at a time; the others go through `keys` (rank_long).
 __global__ __launch_bounds__(256) void fill_kernel(Walk w, const int32_t* __restrict__ dst_ptr, int64_t E, int64_t* keys,
                                                    int64_t* __restrict__ edge_src, int64_t* __restrict__ edge_dst,
                                                    double* __restrict__ edge_shifts) {
@@ -270,7 +313,8 @@ __global__ __launch_bounds__(256) void fill_kernel(Walk w, const int32_t* __rest
   if (end <= beg) return;   // no neighbours, or a segment past a caller's E: the accesses below take deg > 0
   const int32_t deg = (int32_t)(end - beg);
   // the counts came from the same walk, so rank < deg holds unless E cuts the segment: kept as a bound
-  if (deg <= KEY_CAP && w.N < (int64_t)(UINT32_MAX / KEY_IMAGES)) {
+  const bool small_keys = w.N < (int64_t)(UINT32_MAX / KEY_IMAGES);
+  if (deg <= KEY_CAP && small_keys) {
     uint32_t* mine = reinterpret_cast<uint32_t*>(lkeys[wave]);
     if (lane < 4 && (deg & ~3) + lane < KEY_CAP) mine[(deg & ~3) + lane] = UINT32_MAX;
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -292,13 +336,10 @@ __global__ __launch_bounds__(256) void fill_kernel(Walk w, const int32_t* __rest
       if (hit && rank < deg) __hip_atomic_store(keys + beg + rank, key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     });
     __threadfence();
-    for (int32_t t = lane; t < deg; t += 64) {
-      const int64_t key = __hip_atomic_load(keys + beg + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      int32_t rank = 0;
-      for (int32_t q = 0; q < deg; ++q)
-        rank += __hip_atomic_load(keys + beg + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < key;
-      write_edge(beg + rank, key, j, edge_src, edge_dst, edge_shifts);
-    }
+    if (small_keys)
+      rank_long<uint32_t, 4>(keys + beg, deg, lane, lkeys[wave], beg, j, edge_src, edge_dst, edge_shifts);
+    else
+      rank_long<uint64_t, 2>(keys + beg, deg, lane, lkeys[wave], beg, j, edge_src, edge_dst, edge_shifts);
   }
 }
 

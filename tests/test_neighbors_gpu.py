@@ -133,6 +133,15 @@ def test_receivers_around_the_key_capacity(n, r):
     assert deg.max() == n - 1 if r > 8.7 else (deg.max() > 512 and deg.min() < 512)
 
 
+@pytest.mark.parametrize("n", [769, 1024, 1025, 1026, 1600])
+def test_receivers_of_several_key_chunks(n):
+    """More than 512 neighbours: keys ranked 256 at a time against chunks of 512, whole and partial ones."""
+    pos = np.random.default_rng(n).uniform(0.0, 5.0, (n, 3))
+    got = _gpu(pos, np.eye(3) * 100.0, 9.0, pbc=False)
+    _equal(got, _brute(pos, np.eye(3) * 100.0, 9.0, (0, 0, 0)), n)
+    assert (np.diff(got[3]) == n - 1).all()
+
+
 def test_fill_stays_within_a_smaller_edge_count():
     """fsc_neighbor_fill with fewer edges than the list has: receivers before the cut are whole, nothing is written
     at or past it (receivers wholly past it have no room at all), also where more than 512 keys are ranked."""
