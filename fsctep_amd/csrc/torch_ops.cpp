@@ -884,7 +884,7 @@ std::vector<Tensor> neighbor_list(const Tensor& pos_, const Tensor& cell_, doubl
   const int64_t E = dst_ptr.select(0, N).item<int32_t>();
   TORCH_CHECK(E >= 0, "neighbor_list: edge count overflow");
   Tensor src = at::empty({E}, pos.options().dtype(at::kLong)), dst = at::empty({E}, pos.options().dtype(at::kLong));
-  Tensor shifts = at::empty({E, 3}, pos.options()), fill_ws = at::empty({3 * E}, io);
+  Tensor shifts = at::empty({E, 3}, pos.options()), fill_ws = at::empty({2 * E}, io);
   check(fsc_neighbor_fill(N, E, pp, cell.data_ptr<double>(), flags, cutoff, dst_ptr.data_ptr<int32_t>(),
                           ws.data_ptr<int32_t>(), E ? fill_ws.data_ptr<int32_t>() : nullptr,
                           E ? src.data_ptr<int64_t>() : nullptr, E ? dst.data_ptr<int64_t>() : nullptr,

@@ -98,8 +98,10 @@ int fsc_spatial_order(int64_t n_nodes, const float* pos, int32_t* order, int32_t
  * receiver-sorted, then ascending in (src, s).  Unlike torch_cluster's max_num_neighbors there is no cap.
  * pos [N][3] and cell [3][3] are device doubles; pbc is a host array of 3 int32.
  * Two calls: fsc_neighbor_count fills the receiver CSR dst_ptr [N+1] (the caller reads E = dst_ptr[N]),
- * then fsc_neighbor_fill, with the same workspace (fsc_neighbor_workspace int32, left untouched in
- * between) and fill_ws of 3E int32 (8-byte aligned), writes edge_src, edge_dst [E] and edge_shifts [E][3]. */
+ * then fsc_neighbor_fill, with the same arguments and workspace (fsc_neighbor_workspace int32, left untouched
+ * in between; it holds the positions of the count) and fill_ws of 2E int32 (8-byte aligned), writes edge_src,
+ * edge_dst [E] and edge_shifts [E][3].  With n_edges below dst_ptr[N] nothing at or past n_edges is written, and
+ * the receivers whose segments end before it are whole. */
 int fsc_neighbor_workspace(int64_t n_nodes, int64_t* workspace_ints);
 int fsc_neighbor_count(int64_t n_nodes, const double* pos, const double* cell, const int32_t* pbc, double cutoff,
                        int32_t* dst_ptr, int32_t* workspace, hipStream_t stream);

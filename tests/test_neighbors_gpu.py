@@ -162,7 +162,7 @@ def test_fill_stays_within_a_smaller_edge_count():
         for cut in (1, int(ptr[3]), int(ptr[n // 2]) + 1, E - 1, E):
             src = torch.full((E + 1024,), -7, dtype=torch.int64, device=DEV)
             dst, sh = src.clone(), torch.full((E + 1024, 3), -7.0, dtype=torch.float64, device=DEV)
-            fill = torch.empty(3 * E, dtype=torch.int32, device=DEV)
+            fill = torch.empty(2 * E, dtype=torch.int32, device=DEV)
             _lib.call("fsc_neighbor_fill", n, cut, pos.data_ptr(), cell.data_ptr(), pbc, r, dst_ptr.data_ptr(),
                       ws.data_ptr(), fill.data_ptr(), src.data_ptr(), dst.data_ptr(), sh.data_ptr(), st)
             whole = int(ptr[np.searchsorted(ptr, cut, side="right") - 1])   # end of the last whole segment
