@@ -195,7 +195,7 @@ __global__ __launch_bounds__(256, 2) void node_expand_kernel(const float* __rest
                                                              float* __restrict__ S, int64_t n_nodes,
                                                              PathTiles tiles) {
   constexpr int COLS = 65 * C, WCOLS = ne_wcols(C), NT = WCOLS / 16, KS = C / 32;
-  constexpr int NTC = COLS / WCOLS;                  // column tiles (52 or 26)
+  constexpr int NTC = COLS / WCOLS;                  // column tiles (26, 52 or 130)
   constexpr int NCG = (NTC + NE_TPB - 1) / NE_TPB;   // column groups
   constexpr int RT = NE_ROWS / 64;                   // 16-row tiles per wave
   constexpr int RW = C + 8;                          // fp16 per LDS row (padding against bank conflicts)
@@ -338,20 +338,23 @@ __global__ __launch_bounds__(256, 2) void node_expand_kernel(const float* __rest
 // walking 65 K chunks in sequence).  Products are split-fp16 (mfma_x3, fp32 accuracy at 5x the fp32 MFMA
 // rate): the weights come split (bk6 parts h, l, scaled by sw), the dS rows are scaled by their node's
 // power of two (dscale, from edge_message_grad) and split in registers.  The four
-// waves share the path's weights: each 32-column chunk (C x 32 x 3 parts) is loaded once per block
+// waves share the path's weights: each 32-column chunk (C x 32 x 2 parts) is loaded once per block
 // into LDS (double-buffered) while the waves stream their own dS rows a chunk ahead.
 // Transposed product: bk6 rows (a) are the A operand, dS rows the B operand; tile at's A row
 // i is a = (C/4)*(i/4) + 4*at + i%4, so lane (r, q) ends with C/4 consecutive a of one row; lane
 // group q holds chunk columns 8q..8q+7 of both operands.
-constexpr int NEG_ROWS = 256;   // slot rows per block up to C 64
+constexpr int NEG_ROWS = 256;   // slot rows per block up to C 64, and the units the K split goes by
 // Row tiles of a wave: four, two at C 128, whose 4 x 8 accumulator tiles left 76 registers in scratch memory
 // (1,003 nodes: 670 -> 256 us).
 __host__ __device__ constexpr int neg_rt(int C) { return C > 64 ? 2 : 4; }
 __host__ __device__ constexpr int neg_rows(int C) { return 64 * neg_rt(C); }
 constexpr int NEG_KSPLIT_MAX = 16;
 
-// (path, row tile) units of node_expand_grad, and its K parts: a function of N alone, since the
-// workspace holds one partial input gradient per part
+// Units of NEG_ROWS rows of a path, and the K parts of node_expand_grad: a function of N alone, since the workspace
+// holds one partial input gradient per part.  At C 128, whose blocks take half the rows, the units count half the blocks:
+// twice the parts, which the shorter walks gain from more than the partial sums cost (backward of 1,003 nodes, 8 parts
+// 620 us, 4 parts 649; 1,800 nodes 1,101 and 1,196; 2,100 nodes 1,189 and 1,285; 800 and 3,000 nodes 540 and 507, 1,716
+// and 1,686 us the other way).
 inline int neg_tiles(int64_t N) {
   int64_t t = 0;
   for (int p = 0; p < 6; ++p) t += (N * kNumI[kPathL1H[p]] + NEG_ROWS - 1) / NEG_ROWS;
