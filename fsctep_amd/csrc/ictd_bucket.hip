@@ -1444,11 +1444,14 @@ size_t proj_t_lds(const Dims& d, bool do_u, size_t elem) {
   return do_u ? std::max(main, (size_t)4 * MN * PK * elem) : main;
 }
 
-// Tile width of the resident form, 0 where it does not apply: channels within one matrix of 128 x 128, whole
-// elements filling at least 24 of a tile's 32 rows (every K up to 10; 17 rows of 32 at K 17 would double the work).
+// Tile width of the resident form, 0 where it does not apply: channels within one matrix of 128 x 128, an element's K
+// rows within a tile of 32.  Whole elements leave rows of a tile empty (15 of 32 at K 17), which costs less than the
+// other forms.  210,000 rows, resident / others, us, forward, input gradient, gate gradient: 128 channels, K 16 51 / 97,
+// 55 / 80, 56 / 116, K 17 65 / 102, 75 / 82, 88 / 133, K 11 60 / 100, 78 / 83, 84 / 121; 64 channels, K 17 35 / 55,
+// 33 / 49, 38 / 64; 32 channels, K 17 18 / 31, 20 / 33, 35 / 39.
 int resident_width(const Dims& d) {
-  const int eb = 32 / d.K, c = std::max(d.I, d.O);
-  if (d.K > 32 || eb * d.K < 24 || c > 128) return 0;
+  const int c = std::max(d.I, d.O);
+  if (d.K > 32 || c > 128) return 0;
   return c <= 32 ? 2 : c <= 64 ? 4 : 8;
 }
 
@@ -1601,8 +1604,8 @@ int mix_transpose_g(int64_t B, int32_t P, int32_t K, int32_t I, int32_t O, const
       launch_resident<1>(d, t, grad_out, w, nullptr, y, grad_g, accumulate, st);
       return check_launch("bucket mix_transpose_g") ? 2 : 0;
     }
-    // at most half a slice of channels in a launch that does not fill the chip: every wave for itself (4 channels, K 17,
-    // one path, 1,000 elements in 143 workgroups: 8.3 us against 9.3; 10,000 elements: 39 against 28)
+    // at most half a slice of channels in a launch that does not fill the chip: every wave for itself (4 channels, K 64,
+    // one path, 64 elements: 8.2 us against 9.4; 1,000 elements in 500 workgroups: 15 against 13)
     if (d.I > 16 || (int64_t)grid.x * grid.y > 160) {
       mix32_kernel<true><<<grid, 256, 0, st>>>(d, y, w, nullptr, grad_out, grad_g, accumulate);
       return check_launch("bucket mix_transpose_g") ? 2 : 0;
@@ -1654,7 +1657,7 @@ int mix_transpose_y(int64_t B, int32_t P, int32_t K, int32_t I, int32_t O, const
   if (check_launch("bucket transpose_w")) return 2;
   const dim3 grid((unsigned)((B * K + 127) / 128), (unsigned)(P * ((I + 127) / 128)));
   // at most 16 channels on both sides leave most of a slice and of a lane's eight columns empty: every wave for itself
-  // (16 channels, K 17, 20,000 elements: 35 us against 48)
+  // (16 channels, K 64, 20,000 elements: 107 us against 138)
   if constexpr (std::is_same_v<T, float>)
     if (std::max(I, O) > 16) {
       mix32_ty_kernel<<<grid, 256, 0, st>>>(d, grad_out, workspace, gates, grad_y, accumulate);

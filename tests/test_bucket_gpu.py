@@ -97,15 +97,16 @@ def test_mix_ops(case, dt):
 # tile edges: rows straddling elements (K 3, 5, 7, 9 with 128-row blocks), channels past one 128-column block and
 # past a 32-step slice, more row splits than one; factor columns P*K at each 16-wide tile count, channel tails,
 # m2 above and at 8
-# (the weight matrix resident in LDS: I, O <= 128 and a tile of 32 rows at least 24 full, the forward with one path;
-# else slice by slice where that fills the chip and the slices, or every wave for itself: the last row of cases has the
-# forward at 319 and 320 blocks of 128 rows, the gate gradient at 160 and 161, y's gradient at 16 and 20 channels)
+# (the weight matrix resident in LDS: I, O <= 128 and K <= 32, the forward with one path; else slice by slice where that
+# fills the chip and the slices, or every wave for itself: the last cases have the forward at 319 and 320 blocks of 128
+# rows, the gate gradient at 160 and 161, y's gradient at 16 and 20 channels)
 @pytest.mark.parametrize("case", [(43, 1, 3, 132, 132), (129, 1, 1, 32, 4), (19, 3, 7, 100, 260), (128, 2, 5, 28, 128),
                                   (3000, 1, 9, 64, 36), (1, 1, 128, 4, 4), (33, 1, 12, 20, 32), (34, 1, 11, 32, 20),
                                   (65, 1, 13, 64, 60), (7, 1, 32, 128, 124), (9, 1, 33, 124, 128), (4099, 2, 7, 32, 28),
-                                  (1, 1, 1, 4, 4), (2500, 3, 5, 64, 64), (2401, 1, 17, 32, 32), (2402, 2, 17, 64, 20),
-                                  (1120, 1, 17, 16, 16), (1121, 1, 17, 12, 8), (2409, 1, 17, 48, 36),
-                                  (60, 2, 17, 20, 16), (60, 2, 17, 8, 132)])
+                                  (1, 1, 1, 4, 4), (2500, 3, 5, 64, 64), (50, 1, 17, 32, 64), (41, 2, 21, 128, 36),
+                                  (37, 1, 23, 60, 28), (2401, 2, 17, 32, 32), (2402, 2, 17, 64, 20),
+                                  (1238, 1, 33, 48, 36), (480, 1, 33, 16, 16), (481, 1, 33, 12, 8),
+                                  (60, 2, 33, 20, 16), (60, 2, 17, 8, 132)])
 def test_mix_ops_at_tile_edges(case):
     test_mix_ops(case, torch.float32)
 
