@@ -864,12 +864,17 @@ int forward_s(int64_t N, int D, int nC, float scale, const float* t, const float
 
 // largest D whose backward has the registers for the operand pipeline (at D 9 it spills)
 constexpr int GB_PIPE_DMAX = 7;
-// (64-node tile, row block) pairs up to which the small kernel, with four workgroups a pair, is the faster one.
+// (64-node tile, row block) pairs, the row blocks rounded up to the four column blocks of a step, up to which the small
+// kernel, with four workgroups a pair, is the faster one.
 // nC 192, us, large / small, D 1, 3, 5 | 7, 9: 32 nodes (12 pairs) 37 / 12, 36 / 13, 41 / 15 | 33 / 15, 40 / 17;
 // 512 nodes (96) 39 / 17, 38 / 19, 44 / 24 | 36 / 26, 44 / 31; 1,000 nodes (192) 39 / 26, 39 / 33, 46 / 42 | 38 / 43,
 // 47 / 51; 2,000 nodes (384) 41 / 46, 41 / 55, 48 / 70.  nC 384, 256 nodes (96): 75 / 30, 73 / 34, 84 / 41 | 67 / 43,
-// 80 / 50.  The wide D turn earlier: the large kernel takes 64 nodes a workgroup for them as well.
-constexpr int64_t GBS_UNITS = 192, GBS_UNITS_WIDE = 128;
+// 80 / 50.  The wide D turn earlier: the large kernel takes 64 nodes a workgroup for them as well.  At few row blocks the
+// rounding is what the small kernel loses: nC 48 and 96, S 32, 2,000 nodes (128 and 256 pairs), D 3, 5 | 7, 9: 10 / 7,
+// 12 / 10 | 11 / 12, 13 / 16 and 16 / 16, 21 / 21; 1,000 nodes (64 and 128): 9 / 6, 12 / 7 | 11 / 9, 12 / 10 and 16 / 11,
+// 20 / 14 | 19 / 19, 24 / 23; 1,300 nodes, nC 96 (168): 16 / 12, 20 / 16 | 20 / 21, 24 / 26.  S 64, nC 192, D 7, 9: 640
+// nodes (120) 41 / 32, 57 / 39; 700 nodes (132) 42 / 49, 57 / 63.
+constexpr int64_t gbs_units(int D, int S) { return D == 1 ? 256 : D <= 5 ? 192 : S == 64 ? 128 : 120; }
 
 template <int S, bool BLK>
 int backward_s(int64_t N, int D, int nC, float scale, const float* g, const float* t, const float* Wb, float* dt,
@@ -882,7 +887,7 @@ int backward_s(int64_t N, int D, int nC, float scale, const float* g, const floa
   const float* winv = Wb + (int64_t)n_pairs(nC / 16) * 512 * S;
   LaunchTimer tm("gram_backward", st);
   const int64_t stiles = (N + GBS_NODES - 1) / GBS_NODES;
-  if (stiles * (nC / 16) <= (D <= 5 ? GBS_UNITS : GBS_UNITS_WIDE)) {
+  if (stiles * ((nC / 16 + 3) / 4 * 4) <= gbs_units(D, S)) {
     constexpr int R = 4;   // rows a workgroup (8 rows and two column blocks a step measured no gain at D 7 and 9)
 #define FSC_GBS(DD)                                                                                                  \
   backward_small_kernel<DD, S, R, BLK><<<dim3((unsigned)(nC / 16 * (16 / R)), (unsigned)stiles), 256, 0, st>>>(      \

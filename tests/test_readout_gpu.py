@@ -49,10 +49,14 @@ def test_gram_bilinear_matches_reference(N, D, nC, S):
 
 
 # backward for few nodes (4 rows and 4 column blocks a step): node-tile edges at 64, column blocks not a multiple of
-# 4, the last sizes it takes (192 node tiles x row blocks, 128 at D 7 and 9) and the first of the large kernel
+# 4, the last sizes it takes (node tiles x row blocks, the row blocks rounded up to 4: 256 at D 1, 192 at D 3 and 5, 128
+# at D 7 and 9 with 64 outputs, 120 with 32) and the first of the large kernel
 @pytest.mark.parametrize("N,D,nC,S", [(64, 5, 96, 32), (65, 7, 112, 64), (129, 9, 208, 64), (63, 1, 80, 32),
                                       (1024, 3, 192, 32), (1025, 3, 192, 32), (705, 1, 272, 64), (512, 7, 256, 32),
-                                      (513, 7, 256, 32), (460, 9, 272, 64), (1000, 5, 208, 64)])
+                                      (513, 7, 256, 32), (460, 9, 272, 64), (1000, 5, 208, 64),
+                                      (448, 7, 256, 32), (449, 7, 256, 32), (768, 1, 272, 32), (833, 1, 272, 64),
+                                      (576, 3, 272, 32), (577, 5, 272, 64), (1792, 9, 48, 32), (1793, 9, 48, 32),
+                                      (512, 9, 256, 64), (640, 7, 192, 32), (641, 9, 192, 32), (641, 9, 192, 64)])
 def test_gram_bilinear_backward_at_the_kernel_switch(N, D, nC, S):
     test_gram_bilinear_matches_reference(N, D, nC, S)
 
