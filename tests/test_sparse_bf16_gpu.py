@@ -53,6 +53,39 @@ def test_bf16_conv2_op_against_oracle(C):
     assert rel_inf(res[0][0], ref) < 1e-5                 # and the default path is the fp32-accurate one
 
 
+# the message gradient's channel chunks in four parts (up to 256 atoms), two (up to 2,047) and one
+@pytest.mark.parametrize("N,E,C", [(40, 400, 64), (256, 1500, 32), (257, 1500, 64), (2047, 4000, 32), (2048, 4000, 32)])
+def test_bf16_variant_rounds_the_channel_mix_alone(N, E, C):
+    """With operands that bf16 holds (features +-1 in one channel a node, weights and radial values rounded to bf16) the
+    channel mix is exact, so the outputs and the gradients of the radial values and directions, whose products run at
+    fp32 accuracy, agree to 1e-5; the input gradient, which goes through the mix, to the bf16 bound."""
+    from fsctep_amd import ops
+    from fsctep_amd.graph import prepare_graph
+    from test_sparse_gpu import _graph_with_edge_cases
+    g = torch.Generator().manual_seed(N + C)
+    bf = lambda *s: torch.randn(*s, generator=g, dtype=torch.float64).bfloat16().double()
+    src, dst = _graph_with_edge_cases(N, E, 11)
+    E = src.shape[0]
+    x = torch.zeros(N, 13, C, dtype=torch.float64)
+    x[torch.arange(N)[:, None], torch.arange(13), torch.randint(0, C, (N, 1), generator=g)] = \
+        torch.randint(0, 2, (N, 13), generator=g).double() * 2 - 1
+    h, L, b = bf(E, 64), (bf(6 * C * C, 64) / 8), bf(6 * C * C) / 8
+    v = torch.randn(E, 3, generator=g, dtype=torch.float64)
+    n = (v / v.norm(dim=1, keepdim=True)).float().double()
+    order = torch.argsort(dst, stable=True)
+    xo, ho, no = (t.clone().requires_grad_(True) for t in (x, h[order], n[order]))
+    ref = oracle_conv2(xo, ho, no, L, b, src[order], dst[order], N, 1.0 / (E / N))
+    G = torch.randn(ref.shape, generator=g, dtype=torch.float64).float().double()
+    gx, gh, gn = torch.autograd.grad((ref * G).sum(), (xo, ho, no))
+    gr = prepare_graph(src.to(DEV), dst.to(DEV), torch.zeros(E, 3, device=DEV), N)
+    bk1, bk6 = torch.ops.fsctep.sparse_prepare_weights(L.float().to(DEV), b.float().to(DEV), C)
+    xd, hd, nd = (t.float().to(DEV).requires_grad_(True) for t in (x, h[order], n[order]))
+    out = ops.sparse_conv_apply(xd, hd, nd, bk1, bk6, gr, precision=1)
+    dx, dh, dn = torch.autograd.grad(out, (xd, hd, nd), G.float().to(DEV))
+    assert max(rel_inf(a, r) for a, r in ((out.detach(), ref), (dh, gh), (dn, gn))) < 1e-5
+    assert 1e-5 < rel_inf(dx, gx) < TOL_BF16
+
+
 @pytest.mark.parametrize("prec", [0, 1])
 def test_directions_of_any_length(prec):
     """The op takes any direction vectors: lengths from 0 to 50 (dP grows with the length's square), the default path
