@@ -112,16 +112,11 @@ __device__ __forceinline__ void basis_eval(float r, int k, int nb, float rc, int
   }
 }
 
-// logistic sigmoid with the hardware exp2, and the reciprocal by the hardware's (1 ulp) and one Newton step, which gives
-// a division's accuracy for 3 operations instead of 10 (__fdividef compiles to the full division); the kernels are bound
-// by their VALU operations and take 32 (forward) or 48 (backward) of these a lane and tile.  The reciprocal alone is 7 %
-// faster (250,007 edges, hidden + gates: 164 against 175 us; 273 with divisions) but leaves the Gaussian and cosine bases'
-// outputs 0.3 to 0.5 % further from 64 bits than divisions do (Gaussian, hidden: 2.81e-7 against 2.80e-7).  An
-// overflowing exponential gives 1/inf = 0: the step's error term is then 0 inf and counts as -1.
-__device__ __forceinline__ float sigm(float x) {
-  const float d = 1.f + __expf(-x), r = __builtin_amdgcn_rcpf(d);
-  return fmaf(fmaxf(fmaf(-d, r, 1.f), -1.f), r, r);
-}
+// logistic sigmoid with the hardware exp2 and reciprocal (1 ulp each).  The kernels are bound by their VALU
+// operations and take 32 (forward) or 48 (backward) of these a lane and tile: a division instead of the
+// reciprocal is 10 more operations (__fdividef compiles to the full division).  An overflowing exponential
+// gives 1/inf = 0.
+__device__ __forceinline__ float sigm(float x) { return __builtin_amdgcn_rcpf(1.f + __expf(-x)); }
 
 // 1/s of a power of two s = 2^k, |k| <= 126, by its exponent field
 __device__ __forceinline__ float pow2_inverse(float s) { return __uint_as_float(0x7F000000u - __float_as_uint(s)); }
