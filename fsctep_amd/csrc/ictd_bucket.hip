@@ -1577,7 +1577,7 @@ int mix(int64_t B, int32_t P, int32_t K, int32_t I, int32_t O, const T* y, const
   if (B == 0) return 0;
   const dim3 grid((unsigned)((B * K + 127) / 128), (unsigned)((O + 127) / 128));
   if constexpr (std::is_same_v<T, float>) {
-    const int t = P == 1 ? resident_width(d) : 0;   // several paths add up in one product: slice by slice
+    const int t = P == 1 ? resident_width(d) : 0;   // several paths add up in one product: below
     if (t) {
       launch_resident<0>(d, t, y, w, gates, nullptr, out, accumulate, st);
       return check_launch("bucket mix") ? 2 : 0;
